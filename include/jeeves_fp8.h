@@ -233,6 +233,16 @@ int jv_fp8_quantize_swiglu_output(const void* h, int64_t ldh, const uint16_t* h_
 int jv_fp8_tile_weight(const void* codes, int64_t ldc, int64_t N, int64_t K, void* tiled, void* stream);
 int jv_fp8_untile_weight(const void* tiled, int64_t N, int64_t K, void* codes, int64_t ldc, void* stream);
 
+/* Weight intake, FP8Linear.load_weight (inference/fp8.py:164-166): quantize_rows
+ * of a weight x [N, K] (x_bytes 2: bf16, 4: fp32; row stride ldx in elements)
+ * into codes [N, K] (row stride ldc), scales [N] and, unless tiled is NULL, the
+ * tiled layout above, in one pass on `stream`: the same bits as the quantizers
+ * above and jv_fp8_tile_weight. K % 16 == 0 and K <= 16384; tiled also needs
+ * N % 16 == 0 and K % 128 == 0. Rows are 16-byte aligned; the buffers do not
+ * overlap. */
+int jv_fp8_load_weight(const void* x, int64_t ldx, int x_bytes, int64_t N, int64_t K, void* codes, int64_t ldc,
+                       float* scales, void* tiled, void* stream);
+
 /* Dispatch introspection (the role of split_for, inference/fp8.py:105-109):
  * the number of K splits across workgroups the GEMM uses for these sizes on a
  * device with cu_count compute units (1 = no cross-workgroup split; the

@@ -374,6 +374,26 @@ int jv_fp8_tile_weight(const void* codes, int64_t ldc, int64_t N, int64_t K, voi
                     "weight tiling launch");
 }
 
+int jv_fp8_load_weight(const void* x, int64_t ldx, int x_bytes, int64_t N, int64_t K, void* codes, int64_t ldc,
+                       float* scales, void* tiled, void* stream) {
+  if (x_bytes != 2 && x_bytes != 4) return fail(JV_ERR_VALUE, "weights are bf16 (2 bytes) or fp32 (4), got %d", x_bytes);
+  if (N < 0 || N > INT32_MAX || K <= 0 || K > jv::kLoadMaxCols || K % 16)
+    return fail(JV_ERR_VALUE, "loading a weight needs in_features divisible by 16 up to %d, got %lld", jv::kLoadMaxCols,
+                (long long)K);
+  if (tiled && (N % 16 || K % JV_FP8_BLOCK_K))
+    return fail(JV_ERR_VALUE, "tiling needs N divisible by 16 and K by %d, got N=%lld K=%lld", JV_FP8_BLOCK_K, (long long)N,
+                (long long)K);
+  if (N == 0) return JV_OK;
+  if (!aligned16(x) || ldx < K || (ldx * x_bytes) % 16 || !aligned16(codes) || ldc < K || ldc % 16 || !aligned16(tiled))
+    return fail(JV_ERR_VALUE, "loading a weight needs 16-byte aligned rows");
+  if (codes == tiled) return fail(JV_ERR_VALUE, "the two layouts need a buffer each");
+  return hip_status(x_bytes == 2 ? jv::load_rows_bf16((const uint16_t*)x, ldx, N, (int)K, (uint8_t*)codes, ldc, scales,
+                                                      (uint8_t*)tiled, (hipStream_t)stream)
+                                 : jv::load_rows_f32((const float*)x, ldx, N, (int)K, (uint8_t*)codes, ldc, scales,
+                                                     (uint8_t*)tiled, (hipStream_t)stream),
+                    "weight intake launch");
+}
+
 int jv_fp8_untile_weight(const void* tiled, int64_t N, int64_t K, void* codes, int64_t ldc, void* stream) {
   if (N < 0 || N % 16 || K <= 0 || K % JV_FP8_BLOCK_K || N > INT32_MAX || K > INT32_MAX)
     return fail(JV_ERR_VALUE, "untiling needs N divisible by 16 and K by %d, got N=%lld K=%lld", JV_FP8_BLOCK_K, (long long)N,

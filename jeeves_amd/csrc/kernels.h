@@ -271,6 +271,15 @@ hipError_t quant_h_from_maxima(const uint16_t* h, int64_t ldh, const uint16_t* p
 hipError_t quant_rows_f32(const float* x, int64_t ldx, int64_t M, int K, uint8_t* codes, int64_t ldc, float* scales,
                           hipStream_t stream);
 
+// Weight intake (load.hip): codes row-major [N, K] (row stride ldc), scales
+// and, unless null, the tiled copy in one pass; K % 16 == 0 up to
+// kLoadMaxCols, with the tiled copy K % 128 == 0 and N % 16 == 0.
+constexpr int kLoadMaxCols = 16384;
+hipError_t load_rows_bf16(const uint16_t* x, int64_t ldx, int64_t N, int K, uint8_t* codes, int64_t ldc, float* scales,
+                          uint8_t* tiled, hipStream_t stream);
+hipError_t load_rows_f32(const float* x, int64_t ldx, int64_t N, int K, uint8_t* codes, int64_t ldc, float* scales,
+                         uint8_t* tiled, hipStream_t stream);
+
 // swiglu: the plan of a fused SwiGLU gate+up GEMM (a gate/up tile pair per
 // wave, no split-K).
 DecodePlan decode_plan(int64_t M, int64_t N, int64_t K, int cu_count, bool swiglu = false);

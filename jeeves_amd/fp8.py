@@ -568,7 +568,43 @@ class FP8Linear(nn.Module):
 
     @torch.no_grad()
     def load_weight(self, weight: torch.Tensor) -> None:
-        self.load_codes(*quantize_rows(weight.to(self.weight.device)))
+        weight = weight.detach().to(self.weight.device)
+        if not self._load_in_place(weight):
+            self.load_codes(*quantize_rows(weight))
+
+    def _load_in_place(self, weight: torch.Tensor) -> bool:
+        """Quantize ``weight`` straight into ``weight``, ``scale`` and the tiled
+        copy with one kernel (C ABI ``jv_fp8_load_weight``), where it takes the
+        operands: bf16 or fp32 [N,K] with 16-byte aligned rows of at most
+        ``QUANT_MAX_PACKED_COLS`` elements into contiguous buffers of this
+        module's device. The same bits as ``quantize_rows`` and ``load_codes``,
+        which take everything else (and subclasses with a ``load_codes`` of
+        their own)."""
+        codes, scale, tiled = self.weight, self.scale, self.tiled_codes if self.tiled else None
+        N, K = codes.shape
+        dev = codes.device
+        if (type(self).load_codes is not FP8Linear.load_codes or dev.type != "cuda"
+                or weight.dtype not in (torch.bfloat16, torch.float32) or weight.shape != codes.shape
+                or not N or not K or K % 16 or K > QUANT_MAX_PACKED_COLS or codes.dtype != FP8
+                or scale.dtype != torch.float32 or scale.shape != (N,) or not scale.is_contiguous() or scale.device != dev
+                or weight.layout != torch.strided or not _rows_aligned(weight, weight.element_size()) or weight.stride(0) < K
+                or not codes.is_contiguous() or codes.data_ptr() % 16):
+            return False
+        if tiled is not None and (tiled.device != dev or tiled.shape != codes.shape or tiled.element_size() != 1
+                                  or not tiled.is_contiguous() or tiled.data_ptr() % 16):
+            return False
+        with torch.cuda.device(dev):
+            _lib.check(_lib.lib().jv_fp8_load_weight(weight.data_ptr(), weight.stride(0), weight.element_size(), N, K,
+                                                     codes.data_ptr(), K, scale.data_ptr(),
+                                                     tiled.data_ptr() if tiled is not None else None, _stream(dev)))
+        # The kernel's writes count as in-place ones, so that a merged module
+        # over these buffers sees them.
+        for t in (codes, scale):
+            if not torch.is_inference(t):
+                torch.autograd.graph.increment_version(t)
+        if tiled is not None:
+            self._tiled_from = self._weight_key()
+        return True
 
     def set_lora(self, a: torch.Tensor, b: torch.Tensor, scaling: float) -> None:
         """Attach ``y += scaling * (x A^T) B^T`` (A [r,in], B [out,r], bf16)."""
