@@ -261,6 +261,10 @@ int quant_chunks(int K);
 // ldc ignored; the padding rows get zero codes).
 hipError_t quant_rows_bf16(const uint16_t* x, int64_t ldx, int64_t M, int K, uint8_t* codes, int64_t ldc, float* scales,
                            const uint16_t* lora_a, int rank, float* lora_t, bool packed, hipStream_t stream);
+// The same with rank-16 LoRA, two rows per workgroup (quant_lora.hip), for
+// more than kDecodeMaxRows rows of at most 16384 elements.
+hipError_t quant_lora_bf16(const uint16_t* x, int64_t ldx, int64_t M, int K, uint8_t* codes, int64_t ldc, float* scales,
+                           const uint16_t* lora_a, float* lora_t, bool packed, hipStream_t stream);
 hipError_t quant_swiglu_bf16(const uint16_t* gate, int64_t ldg, const uint16_t* up, int64_t ldu, int64_t M, int K,
                              uint8_t* codes, int64_t ldc, float* scales, uint16_t* h_out, int64_t ldh,
                              const uint16_t* lora_a, int rank, float* lora_t, bool packed, hipStream_t stream);
