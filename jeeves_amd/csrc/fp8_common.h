@@ -259,17 +259,18 @@ __device__ __forceinline__ f32x4 mfma_16x16x128_fp8(i32x8 a, i32x8 b, f32x4 c) {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-// 8 e4m3 codes (two dwords) -> 8 bf16 (a 16-byte MFMA operand), in order.
+// 8 e4m3 codes (two dwords) -> 8 bf16 (a 16-byte MFMA operand), in order, by
+// v_cvt_scalef32_pk_bf16_fp8 with scale 1: every e4m3 value is a bf16 value,
+// so nothing rounds. Half the instructions of v_cvt_pk_f32_fp8 and a byte
+// permute of the two upper halves: W8A16 gate+up at 64 / 2048 tokens 39.0 /
+// 377 -> 35.4 / 361 us, down at 96 / 1024 68.0 / 153 -> 59.4 / 135.
 __device__ __forceinline__ bf16x8 e4m3x8_to_bf16(uint32_t lo, uint32_t hi) {
-  typedef float f32x2 __attribute__((ext_vector_type(2)));
-  const f32x2 a = __builtin_amdgcn_cvt_pk_f32_fp8((int)lo, false), b = __builtin_amdgcn_cvt_pk_f32_fp8((int)lo, true);
-  const f32x2 c = __builtin_amdgcn_cvt_pk_f32_fp8((int)hi, false), d = __builtin_amdgcn_cvt_pk_f32_fp8((int)hi, true);
-  // The bf16 value is the upper half of the exact fp32 value.
-  const i32x4 v = {(int)__builtin_amdgcn_perm(__float_as_uint(a.y), __float_as_uint(a.x), 0x07060302),
-                   (int)__builtin_amdgcn_perm(__float_as_uint(b.y), __float_as_uint(b.x), 0x07060302),
-                   (int)__builtin_amdgcn_perm(__float_as_uint(c.y), __float_as_uint(c.x), 0x07060302),
-                   (int)__builtin_amdgcn_perm(__float_as_uint(d.y), __float_as_uint(d.x), 0x07060302)};
-  return __builtin_bit_cast(bf16x8, v);
+  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+  const bf16x2_t a = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, false);
+  const bf16x2_t b = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, true);
+  const bf16x2_t c = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, false);
+  const bf16x2_t d = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, true);
+  return bf16x8{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
 }
 
 __device__ __forceinline__ i32x8 cat8(i32x4 lo, i32x4 hi) {

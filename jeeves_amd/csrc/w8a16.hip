@@ -5,7 +5,7 @@
 // added afterwards in bf16 (inference/fp8.py:183-184).
 //
 // On gfx950 the e4m3 weight bytes become bf16 in registers with
-// v_cvt_pk_f32_fp8 (exact: every e4m3 value is a bf16 value) and feed bf16
+// v_cvt_scalef32_pk_bf16_fp8 (exact: every e4m3 value is a bf16 value) and feed bf16
 // MFMAs with the activations as they are -- no activation quantization, no
 // fp16 detour. Decode (M <= 64) mirrors the FP8 decode kernel: weights are
 // the A side of v_mfma_f32_16x16x32_bf16, each wave streams its k range in
