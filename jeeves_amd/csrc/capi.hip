@@ -126,6 +126,13 @@ int run_gemm(const uint8_t* xq, int64_t ldxq, bool packed_x, const float* sx, co
                     "fp8 prefill GEMM launch");
 }
 
+// The decode plan if the GEMM of these sizes quantizes its activations itself.
+bool quantizes_in_gemm(int64_t M, int64_t N, int64_t K, int64_t lora_rank, int cus, bool swiglu, jv::DecodePlan* plan) {
+  if (lora_rank != 0 || M > jv::kDecodeQuantMaxRows || !jv::fp8_decode_kernel_for(M, N, K, cus)) return false;
+  *plan = jv::decode_plan(M, N, K, cus, swiglu);
+  return jv::fp8_quantizes_in_gemm(M, N, K, cus, *plan);
+}
+
 // ldw = 0 selects the tiled weight layout (tiled_w_offset), which needs
 // whole 16-row tiles; a row-major ldw must cover a row.
 int check_weight(int64_t N, int64_t K, int64_t ldw, const void* w) {
@@ -279,6 +286,12 @@ int jv_fp8_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, const 
   ws += round_up(M * lora_rank * 4, 256);
   const int64_t rest = workspace_bytes - (ws - (uint8_t*)workspace);
   hipStream_t s = (hipStream_t)stream;
+  jv::DecodePlan fused;
+  if (quantizes_in_gemm(M, N, K, lora_rank, cu_count_of(-1), 0 != 0, &fused))
+    return hip_status(jv::gemm_decode_quant((const uint16_t*)x, ldx, (const uint8_t*)w, ldw, (int)M, (int)(N), (int)K, fused,
+                                            jv::Epilogue{nullptr, w_scale, (const uint16_t*)bias, nullptr, nullptr, 0.0f,
+                                                         (uint16_t*)y, ldy, 0, nullptr}, s),
+                      "fp8 quantizing decode GEMM launch");
   if (int rc = hip_status(jv::quant_rows_bf16((const uint16_t*)x, ldx, M, (int)K, codes, K, sx, (const uint16_t*)lora_a,
                                               (int)lora_rank, lora_t, packed, s),
                           "activation quantization launch"))
@@ -500,6 +513,12 @@ int jv_fp8_linear_swiglu(const void* x, int64_t ldx, const void* w, int64_t ldw,
   float* lora_t = lora_rank ? (float*)ws : nullptr;
   ws += round_up(M * lora_rank * 4, 256);
   hipStream_t s = (hipStream_t)stream;
+  jv::DecodePlan fused;
+  if (quantizes_in_gemm(M, 2 * I, K, lora_rank, cu_count_of(-1), I != 0, &fused))
+    return hip_status(jv::gemm_decode_quant((const uint16_t*)x, ldx, (const uint8_t*)w, ldw, (int)M, (int)(2 * I), (int)K, fused,
+                                            jv::Epilogue{nullptr, w_scale, (const uint16_t*)bias, nullptr, nullptr, 0.0f,
+                                                         (uint16_t*)h, ldh, I, h_amax}, s),
+                      "fp8 quantizing decode GEMM launch");
   if (int rc = hip_status(jv::quant_rows_bf16((const uint16_t*)x, ldx, M, (int)K, codes, K, sx, (const uint16_t*)lora_a,
                                               (int)lora_rank, lora_t, true, s),
                           "activation quantization launch"))

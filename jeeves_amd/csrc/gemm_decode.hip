@@ -40,13 +40,24 @@ constexpr int kMaxDecodeSplits = 16;
 // range is its share of the whole row with the compile-time divisor WAVES;
 // with the split count a run-time value the same kernel took 1 us longer
 // at M = 16 on gate+up (19.7 vs 18.7 us), even at one split.
-template <int MT, int RT, int WAVES, int UNROLL, bool PACKX, int RANK, bool PACKW, bool SW = false, bool SPLIT = false>
+// MQ > 0: the workgroup quantizes the activations itself (1 to MQ tokens, MT
+// = 1): xq is then the bf16 rows (ldxq their stride in elements), and NCQ
+// 8-element chunks per lane cover a row shared by WAVES / MQ waves. The row maxima, scales and codes
+// are quant_row's, bit for bit. The rows' loads go out first, the first burst
+// of weights right behind them, so the quantization runs while the weights are
+// on their way; the codes go to LDS, M rows of them, where the packed codes in
+// memory come in whole 16-row tiles (64 KB of L2 reads per workgroup at K =
+// 4096, as much as its weights). A linear saves the quantizer's launch and a
+// dependent kernel boundary: fp8_quantizes_in_gemm (kernels.h) has the times.
+template <int MT, int RT, int WAVES, int UNROLL, bool PACKX, int RANK, bool PACKW, bool SW = false, bool SPLIT = false,
+          int MQ = 0, int NCQ = 1>
 __global__ __launch_bounds__(64 * WAVES) void gemm_decode_kernel(const uint8_t* __restrict__ xq, int64_t ldxq,
                                                                  const uint8_t* __restrict__ w, int64_t ldw, int M, int N,
                                                                  int K, int splits, float* __restrict__ partial,
                                                                  int* __restrict__ counters, Epilogue ep) {
   static_assert(!SW || RT % 2 == 0, "SwiGLU pairs each gate tile with its up tile");
   static_assert(!(SW && SPLIT), "the SwiGLU epilogue keeps whole k ranges");
+  static_assert(MQ == 0 || (MT == 1 && MQ <= WAVES && RANK == 0 && !SPLIT), "quantizing form");
   __shared__ f32x4 red[WAVES][RT * MT][64];
   __shared__ int is_last;
   const int lane = threadIdx.x & 63;
@@ -88,10 +99,22 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_decode_kernel(const uint8_t* 
     wp[rt] = PACKW ? w + pt * ksteps * 2048 + lane * 16
                    : w + (SW ? pt * 16 + li : (int64_t)min(n0 + rt * 16 + li, N - 1)) * ldw + lk;
   }
+  // The quantizing form's rows, ahead of every other load: waiting for them
+  // then leaves the weights in flight. Row wave % MQ to each wave, its chunks
+  // shared by the WAVES / MQ waves of the row.
+  constexpr int QR = MQ > 0 ? MQ : 1, QW = WAVES / QR;
+  const int qrow = wave % QR, qpart = wave / QR;
+  uint4 xr[NCQ];
+  if constexpr (MQ > 0) {
+    const uint16_t* x = reinterpret_cast<const uint16_t*>(xq) + (int64_t)min(qrow, M - 1) * ldxq;
+#pragma unroll
+    for (int i = 0; i < NCQ; ++i)
+      xr[i] = *reinterpret_cast<const uint4*>(x + (int64_t)min(lane + 64 * (qpart + QW * i), (K >> 3) - 1) * 8);
+  }
   const uint8_t* xp[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
-    xp[mt] = PACKX ? xq + (int64_t)mt * ksteps * 2048 + lane * 16 : xq + (int64_t)min(mt * 16 + li, M - 1) * ldxq + lk;
+    xp[mt] = MQ > 0 ? nullptr : PACKX ? xq + (int64_t)mt * ksteps * 2048 + lane * 16 : xq + (int64_t)min(mt * 16 + li, M - 1) * ldxq + lk;
 
   // Each thread's outputs (idx = threadIdx.x + j * 64 WAVES; channel fastest)
   // and their scales and bias, loaded before the weight stream so the
@@ -108,7 +131,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_decode_kernel(const uint8_t* 
       const int idx = min((int)threadIdx.x + j * kThreads, kOut - 1);
       const int t = idx >> 8, e = idx & 255;
       const int m = min((t % MT) * 16 + (e >> 4), M - 1);
-      pre_sx[j] = ep.sx[m];
+      if constexpr (MQ == 0) pre_sx[j] = ep.sx[m];
       if constexpr (SW) {
         const int64_t hc = (int64_t)(group * (RT / 2) + t / MT) * 16 + (e & 15);
         pre_sw[j] = ep.sw[hc];
@@ -136,6 +159,38 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_decode_kernel(const uint8_t* 
   // The burst's addresses are one base per operand plus constant offsets
   // (u steps of 2 KB packed or 128 B row-major), which the loads take as
   // immediates instead of a 64-bit add per step (0.5 us of the 1 us above).
+  // Codes of the quantizing form in LDS, one row every K + kCodePad bytes (the
+  // pad puts the rows of a 16-lane read in different banks).
+  constexpr int kCodePad = 32;
+  extern __shared__ __attribute__((aligned(16))) uint8_t qcodes[];
+  const uint8_t* ql = qcodes + (int64_t)(li % QR) * (K + kCodePad) + lk;
+  i32x4 wa[UNROLL][RT][2];
+  // A short burst repeats its last step, so the loads are unconditional and
+  // the wait for the rows does not take the weights in.
+  auto load_w = [&](int s) {
+    constexpr int WSTEP = PACKW ? 2048 : 128;
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      const int64_t off = (int64_t)min(s + u, max(s_end - 1, 0)) * WSTEP;
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+        wa[u][rt][0] = *reinterpret_cast<const i32x4*>(wp[rt] + off);
+        wa[u][rt][1] = *reinterpret_cast<const i32x4*>(wp[rt] + off + (PACKW ? 1024 : 16));
+      }
+    }
+  };
+  // The MFMAs of a burst on codes from LDS.
+  auto multiply_q = [&](int s, auto full) {
+    constexpr bool FULL = decltype(full)::value;
+    const uint8_t* qb = ql + (int64_t)s * 128;
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      if (!FULL && s + u >= s_end) break;
+      const i32x8 b = cat8(*reinterpret_cast<const i32x4*>(qb + u * 128), *reinterpret_cast<const i32x4*>(qb + u * 128 + 16));
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) acc[rt][0] = mfma_16x16x128_fp8(cat8(wa[u][rt][0], wa[u][rt][1]), b, acc[rt][0]);
+    }
+  };
   auto burst = [&](int s, auto full) {
     constexpr bool FULL = decltype(full)::value;
     constexpr int WSTEP = PACKW ? 2048 : 128, XSTEP = PACKX ? 2048 : 128;
@@ -174,8 +229,53 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_decode_kernel(const uint8_t* 
     }
   };
   int s = s_begin;
-  for (; s + UNROLL <= s_end; s += UNROLL) burst(s, std::true_type{});
-  if (s < s_end) burst(s, std::false_type{});
+  if constexpr (MQ > 0) {
+    __shared__ uint32_t qmax[WAVES];
+    __shared__ float qscale[QR];
+    load_w(s);
+    __builtin_amdgcn_sched_barrier(0);
+    uint32_t am = 0;
+    // a repeated last chunk does not change the maximum
+#pragma unroll
+    for (int i = 0; i < NCQ; ++i) {
+      am = pk_max_u16(am, xr[i].x & 0x7FFF7FFFu);
+      am = pk_max_u16(am, xr[i].y & 0x7FFF7FFFu);
+      am = pk_max_u16(am, xr[i].z & 0x7FFF7FFFu);
+      am = pk_max_u16(am, xr[i].w & 0x7FFF7FFFu);
+    }
+    am = wave_max_u32(max(am & 0xFFFFu, am >> 16));
+    if constexpr (QW > 1) {
+      if (lane == 0) qmax[wave] = am;
+      lds_barrier();
+#pragma unroll
+      for (int p = 0; p < QW; ++p) am = max(am, qmax[qrow + QR * p]);
+      am = __builtin_amdgcn_readfirstlane(am);
+    }
+    const float scale = scale_from_amax_bits(am), rcp = 1.0f / scale;
+    const bool fast = am < 0x7F80u;
+    if (lane == 0 && qpart == 0) qscale[qrow] = scale;
+    uint8_t* qout = qcodes + (int64_t)qrow * (K + kCodePad);
+#pragma unroll
+    for (int i = 0; i < NCQ; ++i) {
+      const int c = lane + 64 * (qpart + QW * i);
+      const uint2 q = encode8(xr[i], scale, rcp, fast);
+      if (c < K >> 3) *reinterpret_cast<uint2*>(qout + c * 8) = q;
+    }
+    lds_barrier();
+    // The thread's outputs' token scales.
+#pragma unroll
+    for (int j = 0; j < kPer; ++j)
+      pre_sx[j] = qscale[min((min((int)threadIdx.x + j * kThreads, kOut - 1) & 255) >> 4, QR - 1)];
+    for (; s + UNROLL <= s_end; s += UNROLL) {
+      multiply_q(s, std::true_type{});
+      if (s + UNROLL < s_end) load_w(s + UNROLL);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (s < s_end) multiply_q(s, std::false_type{});
+  } else {
+    for (; s + UNROLL <= s_end; s += UNROLL) burst(s, std::true_type{});
+    if (s < s_end) burst(s, std::false_type{});
+  }
 
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
@@ -390,6 +490,56 @@ static hipError_t launch_decode_mt(const uint8_t* xq, int64_t ldxq, const uint8_
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
+}
+
+template <int RT, int W, int NCQ, int MQ, bool PACKW, bool SW>
+static hipError_t launch_decode_quant(const uint16_t* x, int64_t ldx, const uint8_t* w, int64_t ldw, int M, int N, int K,
+                                      const DecodePlan& p, const Epilogue& ep, hipStream_t stream) {
+  gemm_decode_kernel<1, RT, W, decode_unroll(1, RT, W), true, 0, PACKW, SW, false, MQ, NCQ>
+      <<<dim3((unsigned)p.groups), dim3(64 * W), (size_t)MQ * (K + 32), stream>>>(
+          reinterpret_cast<const uint8_t*>(x), ldx, w, ldw, M, N, K, 1, nullptr, nullptr, ep);
+  return hipGetLastError();
+}
+
+// NC: 8-element chunks of a row per thread of the workgroup.
+template <int RT, int W, int NC, bool SW>
+static hipError_t launch_decode_quant_m(const uint16_t* x, int64_t ldx, const uint8_t* w, int64_t ldw, int M, int N, int K,
+                                        const DecodePlan& p, const Epilogue& ep, hipStream_t stream) {
+#define JV_DECODE_QUANT(MQ)                                                                                       \
+  return ldw == 0 ? launch_decode_quant<RT, W, NC * MQ, MQ, true, SW>(x, ldx, w, ldw, M, N, K, p, ep, stream)      \
+                  : launch_decode_quant<RT, W, NC * MQ, MQ, false, SW>(x, ldx, w, ldw, M, N, K, p, ep, stream)
+  if (M == 1) JV_DECODE_QUANT(1);
+  if (M == 2) JV_DECODE_QUANT(2);
+  JV_DECODE_QUANT(4);
+#undef JV_DECODE_QUANT
+}
+
+hipError_t gemm_decode_quant(const uint16_t* x, int64_t ldx, const uint8_t* w, int64_t ldw, int M, int N, int K,
+                             const DecodePlan& p, const Epilogue& ep, hipStream_t stream) {
+  if (M < 1 || M > kDecodeQuantMaxRows || K <= 0 || K > 16384 || (K & 127) || p.splits != 1 || (p.rt != 1 && p.rt != 2) ||
+      (p.waves != 4 && p.waves != 8))
+    return hipErrorInvalidValue;
+  if (ep.half && (p.rt != 2 || 2 * ep.half != N || ep.half % 16)) return hipErrorInvalidValue;
+  const int nc = (K / 8 + 64 * p.waves - 1) / (64 * p.waves);
+#define JV_DECODE_QUANT_CASE(RT_, W_, NC_)                                                                      \
+  if (p.rt == RT_ && p.waves == W_ && nc <= NC_) {                                                              \
+    if constexpr (RT_ == 2)                                                                                      \
+      if (ep.half) return launch_decode_quant_m<RT_, W_, NC_, true>(x, ldx, w, ldw, M, N, K, p, ep, stream);     \
+    return launch_decode_quant_m<RT_, W_, NC_, false>(x, ldx, w, ldw, M, N, K, p, ep, stream);                   \
+  }
+  // decode_plan takes 4 waves up to K = 4096 (two chunks per thread), 8 above.
+  JV_DECODE_QUANT_CASE(1, 4, 2)
+  JV_DECODE_QUANT_CASE(2, 4, 2)
+  JV_DECODE_QUANT_CASE(1, 8, 1)
+  JV_DECODE_QUANT_CASE(2, 8, 1)
+  JV_DECODE_QUANT_CASE(1, 8, 2)
+  JV_DECODE_QUANT_CASE(2, 8, 2)
+  JV_DECODE_QUANT_CASE(1, 8, 3)
+  JV_DECODE_QUANT_CASE(2, 8, 3)
+  JV_DECODE_QUANT_CASE(1, 8, 4)
+  JV_DECODE_QUANT_CASE(2, 8, 4)
+#undef JV_DECODE_QUANT_CASE
+  return hipErrorInvalidValue;
 }
 
 hipError_t gemm_decode(const uint8_t* xq, int64_t ldxq, bool packed_x, const uint8_t* w, int64_t ldw, int M, int N, int K,

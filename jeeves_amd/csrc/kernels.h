@@ -291,6 +291,24 @@ hipError_t gemm_decode(const uint8_t* xq, int64_t ldxq, bool packed_x, const uin
                        const DecodePlan& plan, float* partial, int* counters, const Epilogue& ep, int rank,
                        hipStream_t stream);
 
+// The decode GEMM with the per-token quantization of bf16 x in it (no codes, no
+// scales, no workspace); plan without a K split, packed or row-major weights.
+constexpr int kDecodeQuantMaxRows = 4;
+// Where it runs: every workgroup repeats the encode (0.3-0.8 us per token),
+// so few tokens, and at most four workgroups per CU's worth of weight (the
+// lm_head's 7760 groups run in 15 rounds: 155 us with a quantizer launch, 161
+// this way). Measured on MI355X (graphs over rotated weights, us at M = 1 / 2 /
+// 4, quantizer launch + GEMM -> this): k/v 6.3 / 6.3 / 6.3 -> 3.9 / 4.5 / 5.4,
+// q/o 7.5 / 7.8 / 7.8 -> 4.8 / 5.5 / 6.6, merged q/k/v 10.2 / 10.4 / 10.2 ->
+// 7.2 / 7.7 / 8.0, gate+up 21.4 / 21.3 / 20.6 -> 18.8 / 19.4 / 19.3, down 14.3 /
+// 14.3 / 14.5 -> 10.8 / 12.3 / 14.3, 2560 x 9728 13.5 / 13.3 / 13.5 -> 8.4 /
+// 9.5 / 11.4. At 8 tokens k/v and q/o tied and gate+up lost (21.0 vs 27.6).
+inline bool fp8_quantizes_in_gemm(int64_t M, int64_t N, int64_t K, int cu_count, const DecodePlan& plan) {
+  return M <= kDecodeQuantMaxRows && K <= 16384 && plan.splits == 1 && plan.groups <= 4 * (int64_t)cu_count;
+}
+hipError_t gemm_decode_quant(const uint16_t* x, int64_t ldx, const uint8_t* w, int64_t ldw, int M, int N, int K,
+                             const DecodePlan& plan, const Epilogue& ep, hipStream_t stream);
+
 // The batch-decode kernel on a batch_plan plan (no workspace, no counters);
 // ldxq = 0 with packed_x: packed codes; ldw = 0: tiled weights; ep.half != 0:
 // fused SwiGLU (packed codes, a batch_plan(..., swiglu = true) plan).
