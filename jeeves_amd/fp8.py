@@ -25,6 +25,9 @@ synchronisation; outputs and workspaces come from torch's caching allocator
 
 from __future__ import annotations
 
+from contextlib import nullcontext
+from functools import lru_cache
+
 import torch
 import torch.nn as nn
 
@@ -57,8 +60,33 @@ def split_for(N: int, K: int, sms: int) -> int:
     return _lib.lib().jv_fp8_split_for(1, N, K, sms)
 
 
+# The calls below sit on the host path of every linear: a decode GEMM of a few
+# microseconds called eagerly is bound by them (k/v at one token 22 us a call
+# with torch.cuda.device, current_stream and the plan queries each time).
+_CURRENT = nullcontext()
+
+
+def _device_guard(device: torch.device):
+    """``torch.cuda.device(device)``, which costs two device switches even where
+    ``device`` is current."""
+    return _CURRENT if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
+
+
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+@lru_cache(maxsize=4096)
+def _plan(device: torch.device, M: int, N: int, K: int, rank: int) -> tuple[int, int, int]:
+    """(tile counters, workspace bytes of a linear, of a GEMM on codes) for these
+    sizes on ``device``, which is current: functions of the sizes and the
+    device's compute units alone."""
+    L = _lib.lib()
+    sizes = (L.jv_fp8_counters_needed(M, N, K, sm_count(device)), L.jv_fp8_linear_workspace_bytes(M, N, K, rank),
+             L.jv_fp8_gemm_workspace_bytes(M, N, K))
+    if min(sizes[1:]) < 0:
+        _lib.check(_lib.JV_ERR_HIP)
+    return sizes
 
 
 def _stream_counters(device: torch.device) -> torch.Tensor:
@@ -74,8 +102,7 @@ def _stream_counters(device: torch.device) -> torch.Tensor:
     return counters
 
 
-def _tile_counters(device: torch.device, M: int, N: int, K: int) -> torch.Tensor | None:
-    need = _lib.lib().jv_fp8_counters_needed(M, N, K, sm_count(device))
+def _tile_counters(device: torch.device, need: int) -> torch.Tensor | None:
     if need <= 0:
         return None
     counters = _stream_counters(device)
@@ -116,7 +143,7 @@ def _check_operands(dev: torch.device, N: int, weight: torch.Tensor, scale: torc
 def _weight_operand(weight: torch.Tensor, tiled: bool) -> tuple[torch.Tensor, int]:
     """Weight bytes and the C ABI's ldw: the row stride, or 0 for the tiled
     layout (``tile_weight``)."""
-    w = weight.view(torch.uint8)
+    w = weight if weight.dtype == torch.uint8 else weight.view(torch.uint8)
     if tiled:
         if weight.shape[0] % 16 or not w.is_contiguous():
             raise ValueError(f"tiled weights are a contiguous [N, K] buffer with N divisible by 16, got {tuple(weight.shape)}")
@@ -149,7 +176,7 @@ def tile_weight(codes: torch.Tensor) -> torch.Tensor:
     if not _rows_aligned(src, 1):
         src = src.contiguous()
     out = torch.empty(N, K, dtype=torch.uint8, device=codes.device)
-    with torch.cuda.device(codes.device):
+    with _device_guard(codes.device):
         _lib.check(_lib.lib().jv_fp8_tile_weight(src.data_ptr(), src.stride(0), N, K, out.data_ptr(), _stream(codes.device)))
     return out.view(codes.dtype)
 
@@ -164,7 +191,7 @@ def untile_weight(tiled: torch.Tensor) -> torch.Tensor:
         out = src.view(N // 16, K // 128, 2, 4, 16, 16).permute(0, 4, 1, 3, 2, 5).contiguous().view(N, K)
         return out.view(tiled.dtype)
     out = torch.empty(N, K, dtype=torch.uint8, device=tiled.device)
-    with torch.cuda.device(tiled.device):
+    with _device_guard(tiled.device):
         _lib.check(_lib.lib().jv_fp8_untile_weight(src.data_ptr(), N, K, out.data_ptr(), K, _stream(tiled.device)))
     return out.view(tiled.dtype)
 
@@ -178,7 +205,7 @@ def _tile_into(codes: torch.Tensor, out: torch.Tensor) -> None:
         return
     if not _rows_aligned(src, 1):
         src = src.contiguous()
-    with torch.cuda.device(codes.device):
+    with _device_guard(codes.device):
         _lib.check(_lib.lib().jv_fp8_tile_weight(src.data_ptr(), src.stride(0), N, K, out.data_ptr(), _stream(codes.device)))
 
 
@@ -219,13 +246,12 @@ def fp8_matmul(x: torch.Tensor, weight: torch.Tensor, scale: torch.Tensor, *, bi
         return y
     if bias is not None:
         bias = bias.to(torch.bfloat16).contiguous()
-    scale = scale.to(torch.float32).contiguous()
+    if scale.dtype != torch.float32 or not scale.is_contiguous():
+        scale = scale.to(torch.float32).contiguous()
     L = _lib.lib()
-    with torch.cuda.device(dev):
-        counters = _tile_counters(dev, M, N, K)
-        ws_bytes = L.jv_fp8_linear_workspace_bytes(M, N, K, rank)
-        if ws_bytes < 0:
-            _lib.check(_lib.JV_ERR_HIP)
+    with _device_guard(dev):
+        need, ws_bytes, _ = _plan(dev, M, N, K, rank)
+        counters = _tile_counters(dev, need)
         ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
         _lib.check(L.jv_fp8_linear(x.data_ptr(), x.stride(0), w.data_ptr(), ldw, scale.data_ptr(),
                                    bias.data_ptr() if bias is not None else None, a.data_ptr() if rank else None,
@@ -262,7 +288,7 @@ def fp8_matmul_w8a16(x: torch.Tensor, weight: torch.Tensor, scale: torch.Tensor,
         bias = bias.to(torch.bfloat16).contiguous()
     scale = scale.to(torch.float32).contiguous()
     L = _lib.lib()
-    with torch.cuda.device(dev):
+    with _device_guard(dev):
         ws_bytes = L.jv_w8a16_workspace_bytes(M, N, K)
         if ws_bytes < 0:
             _lib.check(_lib.JV_ERR_HIP)
@@ -325,11 +351,9 @@ def fp8_matmul_quantized(xq: torch.Tensor, x_scale: torch.Tensor, weight: torch.
         lora_t = lora_t.to(torch.float32).contiguous()
         lora_b = lora_b.to(torch.bfloat16).contiguous()
     L = _lib.lib()
-    with torch.cuda.device(dev):
-        counters = _tile_counters(dev, M, N, K)
-        ws_bytes = L.jv_fp8_gemm_workspace_bytes(M, N, K)
-        if ws_bytes < 0:
-            _lib.check(_lib.JV_ERR_HIP)
+    with _device_guard(dev):
+        need, _, ws_bytes = _plan(dev, M, N, K, rank)
+        counters = _tile_counters(dev, need)
         ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
         _lib.check(L.jv_fp8_gemm(xq.data_ptr(), 0 if packed_rows is not None else xq.stride(0),
                                  x_scale.to(torch.float32).contiguous().data_ptr(), w.data_ptr(),
@@ -371,7 +395,7 @@ def swiglu_quantize(gate: torch.Tensor, up: torch.Tensor, *, lora_a: torch.Tenso
         lora_a = lora_a.to(torch.bfloat16).contiguous()
         t = torch.empty(M, rank, dtype=torch.float32, device=dev)
     if M:
-        with torch.cuda.device(dev):
+        with _device_guard(dev):
             _lib.check(_lib.lib().jv_fp8_swiglu_quantize(gate.data_ptr(), gate.stride(0), up.data_ptr(), up.stride(0), M, I,
                                                          codes.data_ptr(), 0 if packed else I, scales.data_ptr(),
                                                          h.data_ptr() if h is not None else None, I,
@@ -418,11 +442,9 @@ def gate_up_swiglu(x: torch.Tensor, weight: torch.Tensor, scale: torch.Tensor, *
         bias = bias.to(torch.bfloat16).contiguous() if bias is not None else None
         scale = scale.to(torch.float32).contiguous()
         L = _lib.lib()
-        with torch.cuda.device(dev):
-            counters = _tile_counters(dev, M, N, K)
-            ws_bytes = L.jv_fp8_linear_workspace_bytes(M, N, K, rank)
-            if ws_bytes < 0:
-                _lib.check(_lib.JV_ERR_HIP)
+        with _device_guard(dev):
+            need, ws_bytes, _ = _plan(dev, M, N, K, rank)
+            counters = _tile_counters(dev, need)
             ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
             _lib.check(L.jv_fp8_linear_swiglu(x.data_ptr(), x.stride(0), w.data_ptr(), ldw, scale.data_ptr(),
                                               bias.data_ptr() if bias is not None else None, a.data_ptr() if rank else None,
@@ -463,7 +485,7 @@ def quantize_swiglu_output(h: torch.Tensor, amax: torch.Tensor | None = None, *,
     if amax is not None and (amax.shape != (M, I // 16) or amax.element_size() != 2 or not amax.is_contiguous()):
         raise ValueError(f"amax must be a contiguous 16-bit [{M}, {I // 16}] tensor")
     if M:
-        with torch.cuda.device(dev):
+        with _device_guard(dev):
             _lib.check(_lib.lib().jv_fp8_quantize_swiglu_output(h.data_ptr(), h.stride(0),
                                                                 amax.data_ptr() if amax is not None else None, M, I,
                                                                 codes.data_ptr(), 0 if packed else I, scales.data_ptr(),
@@ -523,7 +545,7 @@ class FP8Linear(nn.Module):
         # Inference tensors (made under torch.inference_mode) keep no version
         # counter: their key is the address alone, and in-place writes to them
         # need retile().
-        w = self.weight
+        w = self._buffers["weight"]
         return w.data_ptr(), (-1 if torch.is_inference(w) else w._version)
 
     def kernel_weight(self) -> tuple[torch.Tensor, bool]:
@@ -533,13 +555,14 @@ class FP8Linear(nn.Module):
         write that bumps its version counter (``copy_``, ``load_state_dict``);
         writes that bypass the counter (through ``weight.data``, or into an
         inference tensor) must be followed by ``retile()``."""
+        buffers = self._buffers  # past Module.__getattr__, twice a call
         if not self.tiled:
-            return self.weight, False
+            return buffers["weight"], False
         key = self._weight_key()
         if self._tiled_from != key:
-            _tile_into(self.weight, self.tiled_codes)
+            _tile_into(buffers["weight"], buffers["tiled_codes"])
             self._tiled_from = key
-        return self.tiled_codes, True
+        return buffers["tiled_codes"], True
 
     @torch.no_grad()
     def retile(self) -> None:
@@ -595,7 +618,7 @@ class FP8Linear(nn.Module):
         if tiled is not None and (tiled.device != dev or tiled.shape != codes.shape or tiled.element_size() != 1
                                   or not tiled.is_contiguous() or tiled.data_ptr() % 16):
             return False
-        with torch.cuda.device(dev):
+        with _device_guard(dev):
             _lib.check(_lib.lib().jv_fp8_load_weight(weight.data_ptr(), weight.stride(0), weight.element_size(), N, K,
                                                      codes.data_ptr(), K, scale.data_ptr(),
                                                      tiled.data_ptr() if tiled is not None else None, _stream(dev)))
@@ -638,15 +661,18 @@ class FP8Linear(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         shape = x.shape
-        x2 = x.reshape(-1, shape[-1]).to(torch.bfloat16)
+        x2 = x if len(shape) == 2 else x.reshape(-1, shape[-1])
+        if x2.dtype != torch.bfloat16:
+            x2 = x2.to(torch.bfloat16)
         if x2.stride(-1) != 1:
             x2 = x2.contiguous()
         w, tiled = self.kernel_weight()
+        scale = self._buffers["scale"]
         if self.activations == "bf16":
-            y = fp8_matmul_w8a16(x2, w, self.scale, bias=self.bias, tiled=tiled)
+            y = fp8_matmul_w8a16(x2, w, scale, bias=self.bias, tiled=tiled)
         else:
-            y = fp8_matmul(x2, w, self.scale, bias=self.bias, lora=self.lora, tiled=tiled)
-        return y.view(*shape[:-1], self.out_features)
+            y = fp8_matmul(x2, w, scale, bias=self.bias, lora=self.lora, tiled=tiled)
+        return y if len(shape) == 2 else y.view(*shape[:-1], self.out_features)
 
 
 class FP8SwiGLU(nn.Module):
