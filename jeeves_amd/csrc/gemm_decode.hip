@@ -167,15 +167,19 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_decode_kernel(const uint8_t* 
   i32x4 wa[UNROLL][RT][2];
   // A short burst repeats its last step, so the loads are unconditional and
   // the wait for the rows does not take the weights in.
+  // Tiled weights: a wave-uniform base per tile and step, one lane offset.
   auto load_w = [&](int s) {
-    constexpr int WSTEP = PACKW ? 2048 : 128;
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
-      const int64_t off = (int64_t)min(s + u, max(s_end - 1, 0)) * WSTEP;
+      const int step = min(s + u, max(s_end - 1, 0));
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
-        wa[u][rt][0] = *reinterpret_cast<const i32x4*>(wp[rt] + off);
-        wa[u][rt][1] = *reinterpret_cast<const i32x4*>(wp[rt] + off + (PACKW ? 1024 : 16));
+        const int lt = min(group * RT + rt, ntiles - 1);
+        const int64_t pt = SW ? swiglu_tile(lt, ep.half) : lt;
+        const uint8_t* p = PACKW ? w + (pt * ksteps + step) * 2048 : wp[rt] + (int64_t)step * 128;
+        const uint32_t l = PACKW ? lane * 16 : 0;
+        wa[u][rt][0] = *reinterpret_cast<const i32x4*>(p + l);
+        wa[u][rt][1] = *reinterpret_cast<const i32x4*>(p + l + (PACKW ? 1024 : 16));
       }
     }
   };
