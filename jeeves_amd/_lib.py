@@ -41,6 +41,7 @@ SIGNATURES: dict[str, tuple] = {
     "jv_fp8_quantize_swiglu_output": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_void_p,
                                               c_void_p, c_int64, c_void_p, c_void_p]),
     "jv_w8a16_workspace_bytes": (c_int64, [c_int64, c_int64, c_int64]),
+    "jv_w8a16_counters_needed": (c_int64, [c_int64, c_int64, c_int64, c_int]),
     "jv_w8a16_linear": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64,
                                 c_int64, c_void_p, c_int64, POINTER(c_int32), c_int64, c_void_p]),
     "jv_fp8_tile_weight": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_void_p]),

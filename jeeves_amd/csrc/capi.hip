@@ -147,6 +147,19 @@ int check_weight(int64_t N, int64_t K, int64_t ldw, const void* w) {
   return JV_OK;
 }
 
+// Workspace of a W8A16 call: the packed activations, then the partials of a K
+// split.
+int64_t w8a16_pack_bytes(int64_t M, int64_t N, int64_t K, int cus) {
+  if (!jv::w8a16_packs(M, N, K, cus) || jv::w8a16_batch_plan(M, N, K, cus, nullptr) || !jv::w8a16_decode_kernel_for(M, N, cus))
+    return 0;
+  return round_up(jv::w8a16_packed_bytes(M, K), 256);
+}
+int64_t w8a16_partial_bytes(int64_t M, int64_t N, int64_t K, int cus) {
+  if (jv::w8a16_batch_plan(M, N, K, cus, nullptr)) return 0;
+  if (jv::w8a16_decode_kernel_for(M, N, cus)) return split_partial_bytes(M, N, K, cus);
+  return round_up(jv::w8a16_prefill_partial_bytes(M, N, K, cus), 256);
+}
+
 int check_lora(int64_t rank, const void* a_or_t, const void* b) {
   if (rank == 0) return JV_OK;
   if (rank != 16) return fail(JV_ERR_VALUE, "LoRA rank %lld is not supported (16 is)", (long long)rank);
@@ -303,9 +316,14 @@ int jv_fp8_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, const 
 int64_t jv_w8a16_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   const int cus = cu_count_of(-1);
   if (cus <= 0) return -1;
-  if (jv::w8a16_batch_plan(M, N, K, cus, nullptr)) return 0;
-  if (jv::w8a16_decode_kernel_for(M, N, cus)) return split_partial_bytes(M, N, K, cus);
-  return round_up(jv::w8a16_prefill_partial_bytes(M, N, K, cus), 256);
+  return w8a16_pack_bytes(M, N, K, cus) + w8a16_partial_bytes(M, N, K, cus);
+}
+
+int64_t jv_w8a16_counters_needed(int64_t M, int64_t N, int64_t K, int cu_count) {
+  if (K <= 0 || N <= 0 || M <= 0 || cu_count <= 0 || jv::w8a16_batch_plan(M, N, K, cu_count, nullptr)) return 0;
+  if (!jv::w8a16_decode_kernel_for(M, N, cu_count)) return jv::w8a16_prefill_counters(M, N, K, cu_count);
+  const jv::DecodePlan p = jv::decode_plan(M, N, K, cu_count);
+  return p.splits > 1 ? p.groups : 0;
 }
 
 int jv_w8a16_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, const float* w_scale, const void* bias,
@@ -320,6 +338,18 @@ int jv_w8a16_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, cons
   if (cus <= 0) return fail(JV_ERR_HIP, "cannot query the device's compute units");
   hipStream_t s = (hipStream_t)stream;
   jv::BatchPlan batch;
+  // The decode kernels read large activations packed; a caller whose workspace
+  // holds the K split's partials alone has them read as they are.
+  const int64_t pack = w8a16_pack_bytes(M, N, K, cus);
+  if (pack && workspace && aligned16(workspace) && workspace_bytes >= pack + w8a16_partial_bytes(M, N, K, cus)) {
+    if (int rc = hip_status(jv::w8a16_pack_x((const uint16_t*)x, ldx, (int)M, (int)K, (uint16_t*)workspace, s),
+                            "W8A16 activation packing launch"))
+      return rc;
+    x = workspace;
+    ldx = 0;
+    workspace = (uint8_t*)workspace + pack;
+    workspace_bytes -= pack;
+  }
   if (jv::w8a16_batch_plan(M, N, K, cus, &batch))
     return hip_status(jv::w8a16_batch((const uint16_t*)x, ldx, (const uint8_t*)w, ldw, (int)M, (int)N, (int)K, batch, w_scale,
                                       (const uint16_t*)bias, (uint16_t*)y, ldy, s),

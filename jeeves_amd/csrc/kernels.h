@@ -296,13 +296,14 @@ hipError_t gemm_decode(const uint8_t* xq, int64_t ldxq, bool packed_x, const uin
 constexpr int kDecodeQuantMaxRows = 4;
 // Where it runs: every workgroup repeats the encode (0.3-0.8 us per token),
 // so few tokens, and at most four workgroups per CU's worth of weight (the
-// lm_head's 7760 groups run in 15 rounds: 155 us with a quantizer launch, 161
-// this way). Measured on MI355X (graphs over rotated weights, us at M = 1 / 2 /
+// lm_head's 7760 groups run in 15 rounds: 155 / 161 us at 1 / 4 tokens with a
+// quantizer launch, 156 / 163 this way). Measured on MI355X (graphs over rotated weights, us at M = 1 / 2 /
 // 4, quantizer launch + GEMM -> this): k/v 6.3 / 6.3 / 6.3 -> 3.9 / 4.5 / 5.4,
 // q/o 7.5 / 7.8 / 7.8 -> 4.8 / 5.5 / 6.6, merged q/k/v 10.2 / 10.4 / 10.2 ->
 // 7.2 / 7.7 / 8.0, gate+up 21.4 / 21.3 / 20.6 -> 18.8 / 19.4 / 19.3, down 14.3 /
 // 14.3 / 14.5 -> 10.8 / 12.3 / 14.3, 2560 x 9728 13.5 / 13.3 / 13.5 -> 8.4 /
-// 9.5 / 11.4. At 8 tokens k/v and q/o tied and gate+up lost (21.0 vs 27.6).
+// 9.5 / 11.4. At 8 tokens, one row per wave, merged q/k/v
+// gains 1.0 us, gate+up 0.2, and down loses 3.4.
 inline bool fp8_quantizes_in_gemm(int64_t M, int64_t N, int64_t K, int cu_count, const DecodePlan& plan) {
   return M <= kDecodeQuantMaxRows && K <= 16384 && plan.splits == 1 && plan.groups <= 4 * (int64_t)cu_count;
 }
@@ -334,6 +335,21 @@ hipError_t w8a16_decode(const uint16_t* x, int64_t ldx, const uint8_t* w, int64_
 hipError_t w8a16_batch(const uint16_t* x, int64_t ldx, const uint8_t* w, int64_t ldw, int M, int N, int K,
                        const BatchPlan& p, const float* sw, const uint16_t* bias, uint16_t* y, int64_t ldy,
                        hipStream_t stream);
+// Rows in the fragment order of w8a16_decode (ldx = 0 there):
+// w8a16_packed_bytes(M, K) bytes. Packing is a launch of its own (2 us), so it
+// pays on large weights past 16 tokens and on all but small ones past 32 (us,
+// graphs over rotated weights, rows as they are vs packed: down M = 24 / 32 /
+// 64 22.6 / 26.6 / 47.6 vs 20.8 / 21.0 / 29.7, merged q/k/v 24 / 48 / 64 11.3 /
+// 16.6 / 20.6 vs 12.8 / 14.6 / 16.4, 5008 x 2560 32 / 48 / 64 8.6 / 11.2 / 13.5
+// vs 8.6 / 9.9 / 11.0; down at 16 tokens 17.3 vs 17.1). The wide weights whose
+// larger batches take prefill tiles (decode_kernel_for) and the batch-decode
+// plans stay without a workspace.
+inline bool w8a16_packs(int64_t M, int64_t N, int64_t K, int cu_count) {
+  return M > 16 && 2 * ((N + 63) / 64) < 3 * (int64_t)cu_count && N * K >= (M > 32 ? int64_t(8) << 20 : int64_t(48) << 20);
+}
+inline int64_t w8a16_packed_bytes(int64_t M, int64_t K) { return (M + 15) / 16 * 16 * K * 2; }
+hipError_t w8a16_pack_x(const uint16_t* x, int64_t ldx, int M, int K, uint16_t* out, hipStream_t stream);
+
 // W8A16 prefill GEMM; `splits` must be w8a16_prefill_splits(M, N, K,
 // cu_count), with w8a16_prefill_partial_bytes of partials and
 // w8a16_prefill_counters zeroed tile counters when above 1.

@@ -32,7 +32,10 @@ __device__ __forceinline__ uint16_t w8a16_out(float acc, float swn, bool has_bia
 // on both operands. SPLIT: workgroups split K (grid.y = splits > 1); without
 // it the wave's k range takes the compile-time divisor W, as in
 // gemm_decode_kernel.
-template <int MT, int RT, int W, int U, bool PACKW, bool SPLIT>
+// PACKX: x holds the rows in fragment order (w8a16_pack_x; ldx unused), one
+// contiguous 1 KB per wave load. Row-major, the 16 rows of a 16-lane group lie
+// apart and each load takes the address unit 64 lookups instead of 8.
+template <int MT, int RT, int W, int U, bool PACKW, bool SPLIT, bool PACKX>
 __global__ __launch_bounds__(64 * W) void w8a16_decode_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                               const uint8_t* __restrict__ w, int64_t ldw, int M, int N,
                                                               int K, int splits, float* __restrict__ partial,
@@ -71,7 +74,9 @@ __global__ __launch_bounds__(64 * W) void w8a16_decode_kernel(const uint16_t* __
                    : w + (int64_t)min(n0 + rt * 16 + li, N - 1) * ldw + j32;
   const uint16_t* xp[MT];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) xp[mt] = x + (int64_t)min(mt * 16 + li, M - 1) * ldx + j32;
+  for (int mt = 0; mt < MT; ++mt)
+    xp[mt] = PACKX ? x + (int64_t)mt * ksteps * 2048 + lane * 8 : x + (int64_t)min(mt * 16 + li, M - 1) * ldx + j32;
+  constexpr int XSTEP = PACKX ? 2048 : 128, XQ = PACKX ? 512 : 8;  // elements per k step, per 32-deep MFMA
 
   // Each thread's output channels (idx = threadIdx.x + j * 64 W; channel
   // fastest) and their scales and bias, loaded before the weight stream so the
@@ -107,7 +112,7 @@ __global__ __launch_bounds__(64 * W) void w8a16_decode_kernel(const uint16_t* __
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) wb[rt] = wp[rt] + (int64_t)s * WSTEP;
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) xb[mt] = xp[mt] + (int64_t)s * 128;
+    for (int mt = 0; mt < MT; ++mt) xb[mt] = xp[mt] + (int64_t)s * XSTEP;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (s + u >= s_end) break;
@@ -119,7 +124,7 @@ __global__ __launch_bounds__(64 * W) void w8a16_decode_kernel(const uint16_t* __
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) xa[u][mt][q] = *reinterpret_cast<const i32x4*>(xb[mt] + u * 128 + 8 * q);
+        for (int q = 0; q < 4; ++q) xa[u][mt][q] = *reinterpret_cast<const i32x4*>(xb[mt] + u * XSTEP + XQ * q);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -375,19 +380,23 @@ static void launch_w8a16_decode(const uint16_t* x, int64_t ldx, const uint8_t* w
                                 uint16_t* y, int64_t ldy, hipStream_t stream) {
   constexpr int U = w8a16_unroll(MT, RT);
   const dim3 grid((unsigned)p.groups, (unsigned)p.splits), block(64 * W);
-#define JV_W8A16_LAUNCH(PW, SP)                                                                                \
-  w8a16_decode_kernel<MT, RT, W, U, PW, SP><<<grid, block, 0, stream>>>(x, ldx, w, ldw, M, N, K, p.splits, partial, \
-                                                                        counters, sw, bias, y, ldy)
+#define JV_W8A16_LAUNCH_X(PW, SP, PX)                                                                              \
+  w8a16_decode_kernel<MT, RT, W, U, PW, SP, PX>                                                                    \
+      <<<grid, block, 0, stream>>>(x, ldx, w, ldw, M, N, K, p.splits, partial, counters, sw, bias, y, ldy)
+#define JV_W8A16_LAUNCH(PW, SP)                    \
+  if (ldx == 0) JV_W8A16_LAUNCH_X(PW, SP, true);   \
+  else JV_W8A16_LAUNCH_X(PW, SP, false)
   // K splits come only with one tile per wave (as in launch_decode).
   if constexpr (RT == 1) {
     if (p.splits > 1) {
-      if (ldw == 0) JV_W8A16_LAUNCH(true, true);
-      else JV_W8A16_LAUNCH(false, true);
+      if (ldw == 0) { JV_W8A16_LAUNCH(true, true); }
+      else { JV_W8A16_LAUNCH(false, true); }
       return;
     }
   }
-  if (ldw == 0) JV_W8A16_LAUNCH(true, false);
-  else JV_W8A16_LAUNCH(false, false);
+  if (ldw == 0) { JV_W8A16_LAUNCH(true, false); }
+  else { JV_W8A16_LAUNCH(false, false); }
+#undef JV_W8A16_LAUNCH_X
 #undef JV_W8A16_LAUNCH
 }
 
@@ -420,6 +429,30 @@ hipError_t w8a16_decode(const uint16_t* x, int64_t ldx, const uint8_t* w, int64_
     case 4: launch_w8a16_decode_mt<4>(x, ldx, w, ldw, M, N, K, p, partial, counters, sw, bias, y, ldy, stream); break;
     default: return hipErrorInvalidValue;
   }
+  return hipGetLastError();
+}
+
+// bf16 rows -> fragment order, 16 bytes per thread: piece q (8 elements) of
+// lane l of 16-row tile t and 128-deep step s at (((t * K / 128) + s) * 4 + q)
+// * 1 KB + 16 l, holding row 16 t + l % 16, k = 128 s + 32 (l / 16) + 8 q. Rows
+// past M repeat the last one (their outputs are never stored).
+__global__ __launch_bounds__(256) void w8a16_pack_kernel(const uint16_t* __restrict__ x, int64_t ldx, int M, int K,
+                                                         uint16_t* __restrict__ out) {
+  const uint32_t per_tile = (uint32_t)K * 2;  // 16-byte pieces of a 16-row tile
+  const uint32_t u = blockIdx.x * 256u + threadIdx.x;
+  const uint32_t tile = blockIdx.y;
+  if (u >= per_tile) return;
+  const uint32_t lane = u & 63, q = (u >> 6) & 3, s = u >> 8;
+  const int row = min((int)(tile * 16 + (lane & 15)), M - 1);
+  const int k = (int)(s * 128 + 32 * (lane >> 4) + 8 * q);
+  *reinterpret_cast<uint4*>(out + ((int64_t)tile * per_tile + u) * 8) =
+      *reinterpret_cast<const uint4*>(x + (int64_t)row * ldx + k);
+}
+
+hipError_t w8a16_pack_x(const uint16_t* x, int64_t ldx, int M, int K, uint16_t* out, hipStream_t stream) {
+  if (M < 1 || K <= 0 || (K & 127)) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)((K * 2 + 255) / 256), (unsigned)((M + 15) / 16));
+  w8a16_pack_kernel<<<grid, dim3(256), 0, stream>>>(x, ldx, M, K, out);
   return hipGetLastError();
 }
 

@@ -292,9 +292,9 @@ def fp8_matmul_w8a16(x: torch.Tensor, weight: torch.Tensor, scale: torch.Tensor,
         ws_bytes = L.jv_w8a16_workspace_bytes(M, N, K)
         if ws_bytes < 0:
             _lib.check(_lib.JV_ERR_HIP)
-        # a workspace means a K split (decode or prefill kernel), which counts
-        # its tiles in; the library checks that they fit the counters
-        counters = _stream_counters(dev) if ws_bytes > 0 else None
+        # only a K split counts its tiles in (the workspace may hold packed
+        # activations alone); the library checks that they fit the counters
+        counters = _stream_counters(dev) if L.jv_w8a16_counters_needed(M, N, K, sm_count(dev)) > 0 else None
         ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
         _lib.check(L.jv_w8a16_linear(x.data_ptr(), x.stride(0), w.data_ptr(), ldw, scale.data_ptr(),
                                      bias.data_ptr() if bias is not None else None, y.data_ptr(), N, M, N, K,
