@@ -11,7 +11,8 @@ kernels of ``libjeeves_fp8.so``, called through its C ABI:
   to fp16 with a power-of-two row scale (``inference/fp8.py:46-58``);
 * the GEMM multiplies e4m3 by e4m3 on the FP8 MFMA units and applies
   ``acc * sx[m] * sw[n]`` (+ bias, + optional LoRA) in its epilogue;
-* 1-16 tokens run the HBM-bound split-K decode kernel; 17-128 tokens the
+* 1-16 tokens run the HBM-bound split-K decode kernel, which quantizes 1-4
+  tokens itself on all but the widest weights; 17-128 tokens the
   batch-decode kernel on weights of up to one round of workgroups at
   K = 4096 / 12288 (whole k ranges of weights in registers, the batch's token
   tiles split across workgroups), else deep-ring 64x64 / 64x128 prefill tiles
