@@ -341,12 +341,13 @@ int jv_w8a16_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, cons
   // The decode kernels read large activations packed; a caller whose workspace
   // holds the K split's partials alone has them read as they are.
   const int64_t pack = w8a16_pack_bytes(M, N, K, cus);
-  if (pack && workspace && aligned16(workspace) && workspace_bytes >= pack + w8a16_partial_bytes(M, N, K, cus)) {
+  const bool packed_x =
+      pack && workspace && aligned16(workspace) && workspace_bytes >= pack + w8a16_partial_bytes(M, N, K, cus);
+  if (packed_x) {
     if (int rc = hip_status(jv::w8a16_pack_x((const uint16_t*)x, ldx, (int)M, (int)K, (uint16_t*)workspace, s),
                             "W8A16 activation packing launch"))
       return rc;
     x = workspace;
-    ldx = 0;
     workspace = (uint8_t*)workspace + pack;
     workspace_bytes -= pack;
   }
@@ -382,7 +383,7 @@ int jv_w8a16_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, cons
                   (long long)need);
     partial = reinterpret_cast<float*>(workspace);
   }
-  return hip_status(jv::w8a16_decode((const uint16_t*)x, ldx, (const uint8_t*)w, ldw, (int)M, (int)N, (int)K, plan, partial,
+  return hip_status(jv::w8a16_decode((const uint16_t*)x, ldx, packed_x, (const uint8_t*)w, ldw, (int)M, (int)N, (int)K, plan, partial,
                                      tile_counters, w_scale, (const uint16_t*)bias, (uint16_t*)y, ldy, s),
                     "W8A16 decode GEMM launch");
 }

@@ -329,13 +329,15 @@ hipError_t gemm_prefill(const uint8_t* xq, int64_t ldx, const uint8_t* w, int64_
 
 // W8A16 parity mode (bf16 activations x e4m3 weights, the reference's own
 // arithmetic): y = bf16(acc * sw[n]), then bf16(y + bias[n]) with a bias.
-hipError_t w8a16_decode(const uint16_t* x, int64_t ldx, const uint8_t* w, int64_t ldw, int M, int N, int K,
+// packed_x: x in the fragment order of w8a16_pack_x (ldx unused), 17 tokens up;
+// otherwise rows ldx elements apart, 0 included (one row for every token).
+hipError_t w8a16_decode(const uint16_t* x, int64_t ldx, bool packed_x, const uint8_t* w, int64_t ldw, int M, int N, int K,
                         const DecodePlan& p, float* partial, int* counters, const float* sw, const uint16_t* bias,
                         uint16_t* y, int64_t ldy, hipStream_t stream);
 hipError_t w8a16_batch(const uint16_t* x, int64_t ldx, const uint8_t* w, int64_t ldw, int M, int N, int K,
                        const BatchPlan& p, const float* sw, const uint16_t* bias, uint16_t* y, int64_t ldy,
                        hipStream_t stream);
-// Rows in the fragment order of w8a16_decode (ldx = 0 there):
+// Rows in the fragment order of w8a16_decode (packed_x there):
 // w8a16_packed_bytes(M, K) bytes. Packing is a launch of its own (2 us), so it
 // pays on large weights past 16 tokens and on all but small ones past 32 (us,
 // graphs over rotated weights, rows as they are vs packed: down M = 24 / 32 /

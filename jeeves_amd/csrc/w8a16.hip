@@ -374,59 +374,66 @@ hipError_t w8a16_batch(const uint16_t* x, int64_t ldx, const uint8_t* w, int64_t
 // of 32 bf16 per step) stay within the register budget without spilling.
 constexpr int w8a16_unroll(int mt, int rt) { return rt + 2 * mt <= 4 ? 4 : 2; }
 
-template <int MT, int RT, int W>
+template <int MT, int RT, int W, bool PACKX>
 static void launch_w8a16_decode(const uint16_t* x, int64_t ldx, const uint8_t* w, int64_t ldw, int M, int N, int K,
                                 const DecodePlan& p, float* partial, int* counters, const float* sw, const uint16_t* bias,
                                 uint16_t* y, int64_t ldy, hipStream_t stream) {
   constexpr int U = w8a16_unroll(MT, RT);
   const dim3 grid((unsigned)p.groups, (unsigned)p.splits), block(64 * W);
-#define JV_W8A16_LAUNCH_X(PW, SP, PX)                                                                              \
-  w8a16_decode_kernel<MT, RT, W, U, PW, SP, PX>                                                                    \
+#define JV_W8A16_LAUNCH(PW, SP)                     \
+  w8a16_decode_kernel<MT, RT, W, U, PW, SP, PACKX>  \
       <<<grid, block, 0, stream>>>(x, ldx, w, ldw, M, N, K, p.splits, partial, counters, sw, bias, y, ldy)
-#define JV_W8A16_LAUNCH(PW, SP)                    \
-  if (ldx == 0) JV_W8A16_LAUNCH_X(PW, SP, true);   \
-  else JV_W8A16_LAUNCH_X(PW, SP, false)
   // K splits come only with one tile per wave (as in launch_decode).
   if constexpr (RT == 1) {
     if (p.splits > 1) {
-      if (ldw == 0) { JV_W8A16_LAUNCH(true, true); }
-      else { JV_W8A16_LAUNCH(false, true); }
+      if (ldw == 0) JV_W8A16_LAUNCH(true, true);
+      else JV_W8A16_LAUNCH(false, true);
       return;
     }
   }
-  if (ldw == 0) { JV_W8A16_LAUNCH(true, false); }
-  else { JV_W8A16_LAUNCH(false, false); }
-#undef JV_W8A16_LAUNCH_X
+  if (ldw == 0) JV_W8A16_LAUNCH(true, false);
+  else JV_W8A16_LAUNCH(false, false);
 #undef JV_W8A16_LAUNCH
 }
 
-template <int MT>
+template <int MT, bool PACKX>
 static void launch_w8a16_decode_mt(const uint16_t* x, int64_t ldx, const uint8_t* w, int64_t ldw, int M, int N, int K,
                                    const DecodePlan& p, float* partial, int* counters, const float* sw,
                                    const uint16_t* bias, uint16_t* y, int64_t ldy, hipStream_t stream) {
   if (p.rt == 2) {
     if (p.waves == 8)
-      launch_w8a16_decode<MT, 2, 8>(x, ldx, w, ldw, M, N, K, p, partial, counters, sw, bias, y, ldy, stream);
+      launch_w8a16_decode<MT, 2, 8, PACKX>(x, ldx, w, ldw, M, N, K, p, partial, counters, sw, bias, y, ldy, stream);
     else
-      launch_w8a16_decode<MT, 2, 4>(x, ldx, w, ldw, M, N, K, p, partial, counters, sw, bias, y, ldy, stream);
+      launch_w8a16_decode<MT, 2, 4, PACKX>(x, ldx, w, ldw, M, N, K, p, partial, counters, sw, bias, y, ldy, stream);
   } else {
     if (p.waves == 8)
-      launch_w8a16_decode<MT, 1, 8>(x, ldx, w, ldw, M, N, K, p, partial, counters, sw, bias, y, ldy, stream);
+      launch_w8a16_decode<MT, 1, 8, PACKX>(x, ldx, w, ldw, M, N, K, p, partial, counters, sw, bias, y, ldy, stream);
     else
-      launch_w8a16_decode<MT, 1, 4>(x, ldx, w, ldw, M, N, K, p, partial, counters, sw, bias, y, ldy, stream);
+      launch_w8a16_decode<MT, 1, 4, PACKX>(x, ldx, w, ldw, M, N, K, p, partial, counters, sw, bias, y, ldy, stream);
   }
 }
 
-hipError_t w8a16_decode(const uint16_t* x, int64_t ldx, const uint8_t* w, int64_t ldw, int M, int N, int K,
+template <int MT>
+static void launch_w8a16_decode_x(const uint16_t* x, int64_t ldx, bool packed_x, const uint8_t* w, int64_t ldw, int M, int N,
+                                  int K, const DecodePlan& p, float* partial, int* counters, const float* sw,
+                                  const uint16_t* bias, uint16_t* y, int64_t ldy, hipStream_t stream) {
+  if (packed_x)
+    launch_w8a16_decode_mt<MT, true>(x, ldx, w, ldw, M, N, K, p, partial, counters, sw, bias, y, ldy, stream);
+  else
+    launch_w8a16_decode_mt<MT, false>(x, ldx, w, ldw, M, N, K, p, partial, counters, sw, bias, y, ldy, stream);
+}
+
+hipError_t w8a16_decode(const uint16_t* x, int64_t ldx, bool packed_x, const uint8_t* w, int64_t ldw, int M, int N, int K,
                         const DecodePlan& p, float* partial, int* counters, const float* sw, const uint16_t* bias,
                         uint16_t* y, int64_t ldy, hipStream_t stream) {
-  if (M < 1 || M > kDecodeMaxRows || (K & 127) || p.splits < 1 || p.splits > 16 || (p.splits > 1 && p.rt != 1))
+  if (M < 1 || M > kDecodeMaxRows || (K & 127) || p.splits < 1 || p.splits > 16 || (p.splits > 1 && p.rt != 1) ||
+      (packed_x && M <= 16))
     return hipErrorInvalidValue;
   switch ((M + 15) / 16) {
-    case 1: launch_w8a16_decode_mt<1>(x, ldx, w, ldw, M, N, K, p, partial, counters, sw, bias, y, ldy, stream); break;
-    case 2: launch_w8a16_decode_mt<2>(x, ldx, w, ldw, M, N, K, p, partial, counters, sw, bias, y, ldy, stream); break;
-    case 3: launch_w8a16_decode_mt<3>(x, ldx, w, ldw, M, N, K, p, partial, counters, sw, bias, y, ldy, stream); break;
-    case 4: launch_w8a16_decode_mt<4>(x, ldx, w, ldw, M, N, K, p, partial, counters, sw, bias, y, ldy, stream); break;
+    case 1: launch_w8a16_decode_mt<1, false>(x, ldx, w, ldw, M, N, K, p, partial, counters, sw, bias, y, ldy, stream); break;
+    case 2: launch_w8a16_decode_x<2>(x, ldx, packed_x, w, ldw, M, N, K, p, partial, counters, sw, bias, y, ldy, stream); break;
+    case 3: launch_w8a16_decode_x<3>(x, ldx, packed_x, w, ldw, M, N, K, p, partial, counters, sw, bias, y, ldy, stream); break;
+    case 4: launch_w8a16_decode_x<4>(x, ldx, packed_x, w, ldw, M, N, K, p, partial, counters, sw, bias, y, ldy, stream); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
