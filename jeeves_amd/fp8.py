@@ -149,9 +149,18 @@ def _weight_operand(weight: torch.Tensor, tiled: bool) -> tuple[torch.Tensor, in
         if weight.shape[0] % 16 or not w.is_contiguous():
             raise ValueError(f"tiled weights are a contiguous [N, K] buffer with N divisible by 16, got {tuple(weight.shape)}")
         return w, 0
-    if not _rows_aligned(w, 1):
-        w = w.contiguous()
-    return w, w.stride(0)
+    return _row_major(w)
+
+
+def _row_major(codes: torch.Tensor) -> tuple[torch.Tensor, int]:
+    """Row-major codes and their row stride for the C ABI, where a stride of 0
+    names the packed layouts: one row broadcast by ``expand`` is copied out to
+    its rows, and a single row passes its length."""
+    if not _rows_aligned(codes, 1):
+        codes = codes.contiguous()
+    if codes.stride(0) == 0 and codes.shape[0] > 1:
+        codes = codes.clone(memory_format=torch.contiguous_format)
+    return codes, codes.stride(0) or codes.shape[1]
 
 
 def tileable(out_features: int, in_features: int) -> bool:
@@ -341,8 +350,9 @@ def fp8_matmul_quantized(xq: torch.Tensor, x_scale: torch.Tensor, weight: torch.
         raise ValueError(f"x_scale needs one value per token row ({M}), got {x_scale.numel()}")
     _check_operands(dev, N, weight, scale, bias, x_scale, lora_t, lora_b)
     xq = xq.view(torch.uint8)
-    if packed_rows is None and not _rows_aligned(xq, 1):
-        xq = xq.contiguous()
+    ldxq = 0
+    if packed_rows is None:
+        xq, ldxq = _row_major(xq)
     w, ldw = _weight_operand(weight, tiled)
     y = torch.empty(M, N, device=dev, dtype=torch.bfloat16)
     if M == 0:
@@ -356,7 +366,7 @@ def fp8_matmul_quantized(xq: torch.Tensor, x_scale: torch.Tensor, weight: torch.
         need, _, ws_bytes = _plan(dev, M, N, K, rank)
         counters = _tile_counters(dev, need)
         ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
-        _lib.check(L.jv_fp8_gemm(xq.data_ptr(), 0 if packed_rows is not None else xq.stride(0),
+        _lib.check(L.jv_fp8_gemm(xq.data_ptr(), ldxq,
                                  x_scale.to(torch.float32).contiguous().data_ptr(), w.data_ptr(),
                                  ldw, scale.to(torch.float32).contiguous().data_ptr(),
                                  bias.data_ptr() if bias is not None else None, lora_t.data_ptr() if rank else None,

@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from jeeves_amd import synthetic
-from jeeves_amd.fp8 import FP8Linear, FP8SwiGLU, fp8_matmul, fp8_matmul_w8a16, tile_weight
+from jeeves_amd.fp8 import FP8Linear, FP8SwiGLU, fp8_matmul, fp8_matmul_quantized, fp8_matmul_w8a16, tile_weight
 from jeeves_amd.fp8_weights import quantize_rows
 
 pytestmark = pytest.mark.gpu
@@ -47,3 +47,17 @@ def test_modules_take_one_row_for_every_token(B, T, activations):
     x = row(hidden, 44).expand(B, T, hidden)
     for m in (gate_up, mlp):
         assert torch.equal(m(x), m(x.contiguous()))
+
+
+@pytest.mark.parametrize("M", [1, 8, 33, 200])
+def test_broadcast_codes(M):
+    """Codes of one row, and weight codes of one row, broadcast over the rows."""
+    N, K = 1040, 2560
+    wq, sw = quantize_rows(synthetic.weight(N, K, 45).cuda())
+    xq, sx = quantize_rows(row(K, 46))
+    x = xq.expand(M, K) if M > 1 else xq.expand(8, K)[:1]
+    want = fp8_matmul_quantized(xq.repeat(M, 1), sx.repeat(M), wq, sw)
+    assert torch.equal(fp8_matmul_quantized(x, sx.repeat(M), wq, sw), want)
+    one = wq[5:6].expand(N, K)
+    assert torch.equal(fp8_matmul_quantized(x, sx.repeat(M), one, sw), fp8_matmul_quantized(x, sx.repeat(M), one.contiguous(), sw))
+    assert torch.equal(fp8_matmul(row(K, 46).expand(M, K), one, sw), fp8_matmul(row(K, 46).expand(M, K), one.contiguous(), sw))

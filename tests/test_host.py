@@ -126,6 +126,25 @@ def test_fp8_matmul_validates_before_launch():
         fp8_matmul(x, w, torch.ones(64), lora=(torch.zeros(8, 256), torch.zeros(64, 8), 2.0))
 
 
+def test_broadcast_codes_are_not_taken_for_packed_ones():
+    """A row stride of 0 names the packed layouts at the C ABI: codes of one
+    row broadcast over the rows get strides of their own, a single row its
+    length, and all others go as they are."""
+    from jeeves_amd.fp8 import _row_major, _weight_operand
+
+    codes = torch.arange(32 * 256, dtype=torch.int64).to(torch.uint8).view(32, 256)
+    for view in (codes[3:4].expand(32, 256), codes[3:4].expand(1, 256), codes[3:4].expand(8, 256)[:1]):
+        for got, ld in (_row_major(view), _weight_operand(view.view(FP8), False)):
+            assert ld == 256 and torch.equal(got, view)
+            assert got.as_strided(view.shape, (ld, 1)).equal(view) if got.shape[0] > 1 else True
+    wide = torch.zeros(32, 512, dtype=torch.uint8)[:, :256]
+    got, ld = _row_major(wide)
+    assert ld == 512 and got.data_ptr() == wide.data_ptr()
+    overlapping = torch.zeros(1024, dtype=torch.uint8).as_strided((32, 256), (16, 1))
+    assert _row_major(overlapping)[1] == 16  # the library takes or refuses it
+    assert _weight_operand(codes.view(FP8), True)[1] == 0
+
+
 def test_operands_must_sit_on_a_hip_device():
     """A host pointer passed to a kernel is a GPU memory fault, so host tensors
     are refused before anything is enqueued (as the reference's Triton
