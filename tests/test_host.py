@@ -113,6 +113,34 @@ def test_tiled_layout_on_host():
     assert not FP8Linear(K, 1000, device="meta").tiled
 
 
+@pytest.mark.parametrize("form", ["buffer", "parameter", "parametrized", "attribute"])
+@pytest.mark.parametrize("tiled", [True, False])
+def test_codes_and_scale_need_not_be_buffers(form, tiled, monkeypatch):
+    """The module reads its codes and scale wherever they are registered: as
+    its buffers, as parameters, through a parametrization, as attributes."""
+    g = torch.Generator().manual_seed(5)
+    N, K = 32 if tiled else 24, 128
+    codes = torch.randint(0, 0x7E, (N, K), generator=g, dtype=torch.uint8).view(FP8)
+    scale = torch.rand(N, generator=g)
+    m = FP8Linear(K, N, device="cpu")
+    m.load_codes(codes, scale)
+    if form == "parameter":
+        m.weight, m.scale = nn.Parameter(codes.clone(), requires_grad=False), nn.Parameter(scale.clone(), requires_grad=False)
+    elif form == "parametrized":
+        nn.utils.parametrize.register_parametrization(m, "weight", nn.Identity(), unsafe=True)
+        nn.utils.parametrize.register_parametrization(m, "scale", nn.Identity(), unsafe=True)
+    elif form == "attribute":
+        del m.weight, m.scale
+        m.weight, m.scale = codes.clone(), scale.clone()
+    want = jeeves_amd.fp8.tile_weight(codes) if tiled else codes
+    got, is_tiled = m.kernel_weight()
+    assert is_tiled == tiled and torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+    seen = []
+    monkeypatch.setattr(jeeves_amd.fp8, "fp8_matmul", lambda x, w, s, **kw: seen.append((w, s)) or torch.zeros(x.shape[0], N))
+    m(torch.zeros(3, K))
+    assert torch.equal(seen[0][0].view(torch.uint8), want.view(torch.uint8)) and torch.equal(seen[0][1], scale)
+
+
 def test_fp8_matmul_validates_before_launch():
     x = torch.zeros(4, 100, dtype=torch.bfloat16)
     w = torch.zeros(64, 100, dtype=torch.uint8).view(FP8)
