@@ -100,7 +100,8 @@ int64_t jv_fp8_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t l
  * ldw = 0: the tiled layout below);
  * w_scale: [N] fp32; bias: [N] bf16 or NULL; lora_a: [rank,K] bf16 and
  * lora_b: [N,rank] bf16, or NULL with lora_rank 0 (rank 16 supported);
- * y: [M,N] bf16 (row stride ldy).
+ * y: [M,N] bf16 (row stride ldy); it may overlap x, all of which is read
+ * before any of y is written, and no other operand.
  * K must be a positive multiple of 128 (JV_ERR_VALUE otherwise, the
  * ValueError of inference/fp8.py:115-117). workspace must hold
  * jv_fp8_linear_workspace_bytes(M,N,K,rank) bytes (256-byte aligned).
@@ -142,7 +143,8 @@ int jv_fp8_linear_noalloc(const void* x, int64_t ldx, const void* w, int64_t ldw
  *   y[m,n] = bf16( sum_k x[m,k] * w[n,k] * w_scale[n] )   (bf16 x e4m3, fp32 sums)
  *   then, with a bias, y[m,n] = bf16( y[m,n] + bias[n] ).
  * No activation quantization: the bf16 activations enter the GEMM as they
- * are. Arguments as jv_fp8_linear (no LoRA); K a positive multiple of 128.
+ * are. Arguments as jv_fp8_linear (no LoRA), but y must not overlap x; K a
+ * positive multiple of 128.
  * workspace: jv_w8a16_workspace_bytes(M,N,K) bytes: the activations packed for
  * the decode kernel (17-64 tokens on large weights), then the split-K
  * partials of the decode kernel or of the prefill kernel's 64x64 tiles (0 for
@@ -194,7 +196,8 @@ int jv_fp8_swiglu_quantize(const void* gate, int64_t ldg, const void* up, int64_
  * tiled layout); w_scale, bias: [2I]; lora_b: [2I, rank]; h: [M, I] bf16 with
  * row stride ldh >= I; h_amax: NULL or [M, I/16] uint16 receiving, per token
  * and 16 channels of h, the largest |h| as a bf16 magnitude pattern (NaN
- * sorts above inf). I a positive multiple of 16, K <= 16384. workspace:
+ * sorts above inf). h and h_amax may overlap x, as y of jv_fp8_linear. I a
+ * positive multiple of 16, K <= 16384. workspace:
  * jv_fp8_linear_workspace_bytes(M, 2I, K, rank) bytes; tile_counters as for
  * jv_fp8_linear: the fused GEMM takes the plain GEMM's plan for the same
  * weight, a K split across workgroups included (the last workgroup of a

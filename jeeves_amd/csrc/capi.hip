@@ -126,11 +126,40 @@ int run_gemm(const uint8_t* xq, int64_t ldxq, bool packed_x, const float* sx, co
                     "fp8 prefill GEMM launch");
 }
 
+// Whether any of M rows of `bytes` bytes, `ld` bytes apart from p, meets one of
+// M rows of the other.
+bool rows_overlap(const void* p, int64_t ld, int64_t bytes, const void* q, int64_t ldq, int64_t bytes_q, int64_t M) {
+  for (int64_t i = 0; i < M; ++i)
+    for (int64_t j = 0; j < M; ++j) {
+      const uintptr_t a = (uintptr_t)p + i * ld, b = (uintptr_t)q + j * ldq;
+      if (a < b + bytes_q && b < a + bytes) return true;
+    }
+  return false;
+}
+
 // The decode plan if the GEMM of these sizes quantizes its activations itself.
 bool quantizes_in_gemm(int64_t M, int64_t N, int64_t K, int64_t lora_rank, int cus, bool swiglu, jv::DecodePlan* plan) {
   if (lora_rank != 0 || M > jv::kDecodeQuantMaxRows || !jv::fp8_decode_kernel_for(M, N, K, cus)) return false;
   *plan = jv::decode_plan(M, N, K, cus, swiglu);
   return jv::fp8_quantizes_in_gemm(M, N, K, cus, *plan);
+}
+
+// Enqueues the quantizing decode GEMM where these sizes take it (*done), with
+// ep.half != 0 for the fused SwiGLU. Its workgroups read x while others store
+// their outputs already, so outputs that overlap x stay with the quantizer
+// launch, which has read all of x before any GEMM workgroup stores.
+int run_quantizing_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, int64_t M, int64_t N, int64_t K,
+                        int64_t lora_rank, const jv::Epilogue& ep, hipStream_t stream, bool* done) {
+  const int cus = cu_count_of(-1);
+  if (cus <= 0) return fail(JV_ERR_HIP, "cannot query the device's compute units");
+  jv::DecodePlan plan;
+  *done = quantizes_in_gemm(M, N, K, lora_rank, cus, ep.half != 0, &plan) &&
+          !rows_overlap(x, ldx * 2, K * 2, ep.y, ep.ldy * 2, (ep.half ? ep.half : N) * 2, M) &&
+          !(ep.parts && rows_overlap(x, ldx * 2, K * 2, ep.parts, ep.half / 16 * 2, ep.half / 16 * 2, M));
+  if (!*done) return JV_OK;
+  return hip_status(jv::gemm_decode_quant((const uint16_t*)x, ldx, (const uint8_t*)w, ldw, (int)M, (int)N, (int)K, plan, ep,
+                                          stream),
+                    "fp8 quantizing decode GEMM launch");
 }
 
 // ldw = 0 selects the tiled weight layout (tiled_w_offset), which needs
@@ -299,12 +328,9 @@ int jv_fp8_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, const 
   ws += round_up(M * lora_rank * 4, 256);
   const int64_t rest = workspace_bytes - (ws - (uint8_t*)workspace);
   hipStream_t s = (hipStream_t)stream;
-  jv::DecodePlan fused;
-  if (quantizes_in_gemm(M, N, K, lora_rank, cu_count_of(-1), 0 != 0, &fused))
-    return hip_status(jv::gemm_decode_quant((const uint16_t*)x, ldx, (const uint8_t*)w, ldw, (int)M, (int)(N), (int)K, fused,
-                                            jv::Epilogue{nullptr, w_scale, (const uint16_t*)bias, nullptr, nullptr, 0.0f,
-                                                         (uint16_t*)y, ldy, 0, nullptr}, s),
-                      "fp8 quantizing decode GEMM launch");
+  bool done;
+  const jv::Epilogue ep{nullptr, w_scale, (const uint16_t*)bias, nullptr, nullptr, 0.0f, (uint16_t*)y, ldy, 0, nullptr};
+  if (int rc = run_quantizing_gemm(x, ldx, w, ldw, M, N, K, lora_rank, ep, s, &done); rc || done) return rc;
   if (int rc = hip_status(jv::quant_rows_bf16((const uint16_t*)x, ldx, M, (int)K, codes, K, sx, (const uint16_t*)lora_a,
                                               (int)lora_rank, lora_t, packed, s),
                           "activation quantization launch"))
@@ -544,12 +570,9 @@ int jv_fp8_linear_swiglu(const void* x, int64_t ldx, const void* w, int64_t ldw,
   float* lora_t = lora_rank ? (float*)ws : nullptr;
   ws += round_up(M * lora_rank * 4, 256);
   hipStream_t s = (hipStream_t)stream;
-  jv::DecodePlan fused;
-  if (quantizes_in_gemm(M, 2 * I, K, lora_rank, cu_count_of(-1), I != 0, &fused))
-    return hip_status(jv::gemm_decode_quant((const uint16_t*)x, ldx, (const uint8_t*)w, ldw, (int)M, (int)(2 * I), (int)K, fused,
-                                            jv::Epilogue{nullptr, w_scale, (const uint16_t*)bias, nullptr, nullptr, 0.0f,
-                                                         (uint16_t*)h, ldh, I, h_amax}, s),
-                      "fp8 quantizing decode GEMM launch");
+  bool done;
+  const jv::Epilogue ep{nullptr, w_scale, (const uint16_t*)bias, nullptr, nullptr, 0.0f, (uint16_t*)h, ldh, I, h_amax};
+  if (int rc = run_quantizing_gemm(x, ldx, w, ldw, M, 2 * I, K, lora_rank, ep, s, &done); rc || done) return rc;
   if (int rc = hip_status(jv::quant_rows_bf16((const uint16_t*)x, ldx, M, (int)K, codes, K, sx, (const uint16_t*)lora_a,
                                               (int)lora_rank, lora_t, true, s),
                           "activation quantization launch"))

@@ -119,3 +119,16 @@ def test_noalloc_refuses_sizes_beyond_its_scratch():
         assert rc == _lib.JV_ERR_VALUE and b"needs" in L.jv_fp8_last_error(), (M, K)
     assert L.jv_fp8_linear_workspace_bytes(8176, 4096, 4096, 0) <= limit - 16384
     assert L.jv_fp8_linear_workspace_bytes(2720, 4096, 12288, 0) <= limit - 16384
+
+
+@pytest.mark.parametrize("M", [1, 3, 4, 5])
+def test_noalloc_over_its_activations(M):
+    """y over x's own rows: all of x is read before y is written."""
+    N = K = 4096
+    wq, sw = quantize_rows(synthetic.weight(N, K, 50).cuda())
+    w = tile_weight(wq)
+    x = synthetic.activations_outliers(M, K, 51 + M).cuda()
+    want = with_workspace(x, w, 0, sw, None, None, N)
+    _lib.check(_lib.lib().jv_fp8_linear_noalloc(x.data_ptr(), K, w.data_ptr(), 0, sw.data_ptr(), None, None, None, 0, 0.0,
+                                                x.data_ptr(), N, M, N, K, torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(x, want)
