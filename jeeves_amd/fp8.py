@@ -620,12 +620,18 @@ class FP8Linear(nn.Module):
         operands: bf16 or fp32 [N,K] with 16-byte aligned rows of at most
         ``QUANT_MAX_PACKED_COLS`` elements into contiguous buffers of this
         module's device. The same bits as ``quantize_rows`` and ``load_codes``,
-        which take everything else (and subclasses with a ``load_codes`` of
-        their own)."""
-        codes, scale, tiled = self.weight, self.scale, self.tiled_codes if self.tiled else None
+        which take everything else: a ``load_codes`` that is not this class's,
+        codes or a scale that are not the buffers (the result of a
+        parametrization, say), inference tensors outside inference mode, which
+        ``copy_`` refuses to write, and a weight whose memory the kernel's own
+        writes would change, or that torch negates on reading."""
+        codes, scale = self._buffers.get("weight"), self._buffers.get("scale")
+        tiled = self._buffers.get("tiled_codes") if self.tiled else None
+        if codes is None or scale is None or (self.tiled and tiled is None):
+            return False
         N, K = codes.shape
         dev = codes.device
-        if (type(self).load_codes is not FP8Linear.load_codes or dev.type != "cuda"
+        if (getattr(self.load_codes, "__func__", None) is not FP8Linear.load_codes or dev.type != "cuda" or weight.is_neg()
                 or weight.dtype not in (torch.bfloat16, torch.float32) or weight.shape != codes.shape
                 or not N or not K or K % 16 or K > QUANT_MAX_PACKED_COLS or codes.dtype != FP8
                 or scale.dtype != torch.float32 or scale.shape != (N,) or not scale.is_contiguous() or scale.device != dev
@@ -634,6 +640,12 @@ class FP8Linear(nn.Module):
             return False
         if tiled is not None and (tiled.device != dev or tiled.shape != codes.shape or tiled.element_size() != 1
                                   or not tiled.is_contiguous() or tiled.data_ptr() % 16):
+            return False
+        if not torch.is_inference_mode_enabled() and (torch.is_inference(codes) or torch.is_inference(scale)):
+            return False
+        first, last = weight.data_ptr(), weight.data_ptr() + ((N - 1) * weight.stride(0) + K) * weight.element_size()
+        if any(t.data_ptr() < last and first < t.data_ptr() + t.numel() * t.element_size()
+               for t in (codes, scale, tiled) if t is not None):
             return False
         with _device_guard(dev):
             _lib.check(_lib.lib().jv_fp8_load_weight(weight.data_ptr(), weight.stride(0), weight.element_size(), N, K,

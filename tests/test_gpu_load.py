@@ -84,6 +84,64 @@ def test_load_weight_into_a_part_reaches_the_merged_module():
     assert torch.equal(merged(x)[:, 32:], alone(x))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("where", ["weight", "scale", "tiled_codes"])
+def test_load_weight_from_memory_of_its_own_buffers(where, dtype):
+    """The checkpoint's weight may lie where the module keeps its codes: it is
+    read before anything is written."""
+    N, K = 512, 4096
+    w = synthetic.weight(N, K, 32).to(dtype).cuda()
+    want = FP8Linear(K, N, device="cuda")
+    want.load_weight(w)
+    pool = torch.zeros(N * K * 8, dtype=torch.uint8, device="cuda")
+    m = FP8Linear(K, N, device="cuda")
+    own = getattr(m, where)
+    n = own.numel() * own.element_size()
+    m._buffers[where] = pool[1024:1024 + n].view(own.dtype).view(own.shape)
+    given = pool[:N * K * w.element_size()].view(dtype).view(N, K)
+    given.copy_(w)
+    m.load_weight(given)
+    assert torch.equal(m.weight.view(torch.uint8), want.weight.view(torch.uint8)) and torch.equal(m.scale, want.scale)
+    assert torch.equal(m.kernel_weight()[0], want.kernel_weight()[0])
+
+
+def test_load_weight_leaves_other_tensors_to_load_codes():
+    """Calls that load_codes alone may answer: its override on an instance, a
+    parametrized weight, inference tensors outside inference mode (refused),
+    a weight that torch negates on reading."""
+    N, K = 64, 1024
+    w = synthetic.weight(N, K, 33).cuda()
+    want = FP8Linear(K, N, device="cuda")
+    want.load_weight(w)
+
+    m = FP8Linear(K, N, device="cuda")
+    seen = []
+    m.load_codes = lambda codes, scale: seen.append((codes, scale))
+    m.load_weight(w)
+    assert torch.equal(seen[0][0].view(torch.uint8), want.weight.view(torch.uint8)) and torch.equal(seen[0][1], want.scale)
+
+    class Flip(torch.nn.Module):
+        def forward(self, codes):
+            return (codes.view(torch.uint8) ^ 0x80).view(codes.dtype)
+
+    m = FP8Linear(K, N, device="cuda")
+    m.load_weight(w)
+    torch.nn.utils.parametrize.register_parametrization(m, "weight", Flip(), unsafe=True)
+    m.load_weight(w * 2)  # written to the parametrization's result, which nothing keeps
+    assert torch.equal(m.kernel_weight()[0], tile_weight(want.weight.view(torch.uint8) ^ 0x80))
+
+    with torch.inference_mode():
+        m = FP8Linear(K, N, device="cuda")
+        m.load_weight(w)
+        assert torch.equal(m.weight.view(torch.uint8), want.weight.view(torch.uint8))
+    with pytest.raises(RuntimeError, match="[Ii]nference"):
+        m.load_weight(w)
+
+    m = FP8Linear(K, N, device="cuda")
+    m.load_weight(torch._neg_view(w.float()))
+    assert torch.equal(m.weight.view(torch.uint8) ^ 0x80, want.weight.view(torch.uint8))
+
+
 def test_load_weight_refuses_what_it_cannot_take():
     L, buf = _lib.lib(), torch.zeros(64 * 256, dtype=torch.uint8, device="cuda")
     p = buf.data_ptr()
