@@ -261,6 +261,12 @@ int jv_fp8_load_weight(const void* x, int64_t ldx, int x_bytes, int64_t N, int64
 int jv_fp8_split_for(int64_t M, int64_t N, int64_t K, int cu_count);
 int64_t jv_fp8_counters_needed(int64_t M, int64_t N, int64_t K, int cu_count);
 
+/* 1 if jv_fp8_linear (swiglu != 0: jv_fp8_linear_swiglu with N = 2 I) without
+ * LoRA quantizes its activations inside the GEMM's launch for these sizes
+ * (tiled: ldw = 0), where that is the faster, else 0: a quantizer launch, then
+ * the GEMM. */
+int jv_fp8_quantizes_in_gemm(int64_t M, int64_t N, int64_t K, int tiled, int swiglu, int cu_count);
+
 /* The same introspection for the whole launch: shape[0] = the GEMM kernel
  * (0 decode, 1 prefill lockstep tiles, 2 prefill ping-pong tiles, 3 batch-decode
  * kernel: 17-128 tokens, no K split, no counters), shape[1] =

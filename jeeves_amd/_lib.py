@@ -49,6 +49,7 @@ SIGNATURES: dict[str, tuple] = {
     "jv_fp8_load_weight": (c_int, [c_void_p, c_int64, c_int, c_int64, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_void_p]),
     "jv_fp8_split_for": (c_int, [c_int64, c_int64, c_int64, c_int]),
     "jv_fp8_counters_needed": (c_int64, [c_int64, c_int64, c_int64, c_int]),
+    "jv_fp8_quantizes_in_gemm": (c_int, [c_int64, c_int64, c_int64, c_int, c_int, c_int]),
     "jv_fp8_launch_shape": (c_int, [c_int64, c_int64, c_int64, c_int, POINTER(c_int32)]),
 }
 

@@ -138,10 +138,11 @@ bool rows_overlap(const void* p, int64_t ld, int64_t bytes, const void* q, int64
 }
 
 // The decode plan if the GEMM of these sizes quantizes its activations itself.
-bool quantizes_in_gemm(int64_t M, int64_t N, int64_t K, int64_t lora_rank, int cus, bool swiglu, jv::DecodePlan* plan) {
-  if (lora_rank != 0 || M > jv::kDecodeQuantMaxRows || !jv::fp8_decode_kernel_for(M, N, K, cus)) return false;
+bool quantizes_in_gemm(int64_t M, int64_t N, int64_t K, bool tiled, int64_t lora_rank, int cus, bool swiglu,
+                       jv::DecodePlan* plan) {
+  if (lora_rank != 0 || M > jv::kDecodeQuantMaxRows) return false;
   *plan = jv::decode_plan(M, N, K, cus, swiglu);
-  return jv::fp8_quantizes_in_gemm(M, N, K, cus, *plan);
+  return jv::fp8_quantizes_in_gemm(M, K, tiled, cus, *plan);
 }
 
 // Enqueues the quantizing decode GEMM where these sizes take it (*done), with
@@ -153,7 +154,7 @@ int run_quantizing_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, 
   const int cus = cu_count_of(-1);
   if (cus <= 0) return fail(JV_ERR_HIP, "cannot query the device's compute units");
   jv::DecodePlan plan;
-  *done = quantizes_in_gemm(M, N, K, lora_rank, cus, ep.half != 0, &plan) &&
+  *done = quantizes_in_gemm(M, N, K, ldw == 0, lora_rank, cus, ep.half != 0, &plan) &&
           !rows_overlap(x, ldx * 2, K * 2, ep.y, ep.ldy * 2, (ep.half ? ep.half : N) * 2, M) &&
           !(ep.parts && rows_overlap(x, ldx * 2, K * 2, ep.parts, ep.half / 16 * 2, ep.half / 16 * 2, M));
   if (!*done) return JV_OK;
@@ -480,6 +481,12 @@ int jv_fp8_split_for(int64_t M, int64_t N, int64_t K, int cu_count) {
   if (jv::batch_plan(M, N, K, cu_count, false, nullptr)) return 1;
   if (!jv::fp8_decode_kernel_for(M, N, K, cu_count)) return jv::prefill_tile(M, N, K, cu_count).splits;
   return jv::decode_plan(M, N, K, cu_count).splits;
+}
+
+int jv_fp8_quantizes_in_gemm(int64_t M, int64_t N, int64_t K, int tiled, int swiglu, int cu_count) {
+  if (K <= 0 || K % JV_FP8_BLOCK_K || N <= 0 || M <= 0 || cu_count <= 0) return 0;
+  jv::DecodePlan plan;
+  return quantizes_in_gemm(M, N, K, tiled != 0, 0, cu_count, swiglu != 0, &plan);
 }
 
 int64_t jv_fp8_counters_needed(int64_t M, int64_t N, int64_t K, int cu_count) {

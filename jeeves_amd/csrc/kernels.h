@@ -294,18 +294,55 @@ hipError_t gemm_decode(const uint8_t* xq, int64_t ldxq, bool packed_x, const uin
 // The decode GEMM with the per-token quantization of bf16 x in it (no codes, no
 // scales, no workspace); plan without a K split, packed or row-major weights.
 constexpr int kDecodeQuantMaxRows = 4;
-// Where it runs: every workgroup repeats the encode (0.3-0.8 us per token),
-// so few tokens, and at most four workgroups per CU's worth of weight (the
-// lm_head's 7760 groups run in 15 rounds: 155 / 161 us at 1 / 4 tokens with a
-// quantizer launch, 156 / 163 this way). Measured on MI355X (graphs over rotated weights, us at M = 1 / 2 /
-// 4, quantizer launch + GEMM -> this): k/v 6.3 / 6.3 / 6.3 -> 3.9 / 4.5 / 5.4,
-// q/o 7.5 / 7.8 / 7.8 -> 4.8 / 5.5 / 6.6, merged q/k/v 10.2 / 10.4 / 10.2 ->
-// 7.2 / 7.7 / 8.0, gate+up 21.4 / 21.3 / 20.6 -> 18.8 / 19.4 / 19.3, down 14.3 /
-// 14.3 / 14.5 -> 10.8 / 12.3 / 14.3, 2560 x 9728 13.5 / 13.3 / 13.5 -> 8.4 /
-// 9.5 / 11.4. At 8 tokens, one row per wave, merged q/k/v
-// gains 1.0 us, gate+up 0.2, and down loses 3.4.
-inline bool fp8_quantizes_in_gemm(int64_t M, int64_t N, int64_t K, int cu_count, const DecodePlan& plan) {
-  return M <= kDecodeQuantMaxRows && K <= 16384 && plan.splits == 1 && plan.groups <= 4 * (int64_t)cu_count;
+// Where it runs. It saves the quantizer's launch and a dependent boundary
+// (2.3-4.5 us), and pays in every workgroup: the encode of the rows (per
+// workgroup and token, whatever the weight's width) and the burst of weights
+// issued ahead of it, whose steps past a wave's k range repeat its last one (a
+// wave of K = 5120 has 5 steps and issues 8; row-major, each repeats 64 line
+// lookups). So it wins with few tokens, few rounds of workgroups and bursts
+// that are mostly whole, and loses on short rows of wide weights. The lines
+// below lie where 3600 timed pairs on MI355X cross (1, 2 and 4 tokens, 24 row
+// lengths, 15 widths, plain and SwiGLU; quantizer launch + GEMM against this,
+// us, graphs over 1 GiB of rotated weights, N x K; 3 tokens run the kernel of
+// 4). Tiled weights:
+//   1-2 tokens: 24576 x 4096 at 1 20.8 -> 18.4, 20480 x 2048 at 2 12.3 -> 10.6;
+//     below K = 2048 up to 4 CUs' worth of tiles per token: 20480 x 1024 at 2
+//     8.9 -> 9.5, 24576 x 512 at 1 7.2 -> 7.5.
+//   3-4 tokens, one round: 4096 x 12288 14.5 -> 14.1, past that 4096 x 14336
+//     16.3 -> 17.0; 6144 x 2048 7.1 -> 5.9, 4096 x 1536 5.5 -> 4.9, below that
+//     1024 x 768 4.4 -> 4.4 and, two tiles per wave, SwiGLU 8192 x 1024 6.0 -> 6.2.
+//   3-4 tokens, more rounds, one tile per wave: 12288 x 6144 18.7 -> 18.3, with
+//     repeated steps 12288 x 5120 16.3 -> 16.7; two tiles: 24576 x 4096
+//     21.0 -> 19.4, 32768 x 8192 55.6 -> 51.9, but 24576 x 5120 25.6 -> 26.5 and
+//     24576 x 12288 56.1 -> 59.5.
+// Row-major weights:
+//   1-2 tokens: one tile per wave 4096 x 12288 at 1 16.1 -> 13.1, several
+//     rounds of short rows 8208 x 1024 +12 %; two tiles: 8192 x 4096 at 1 12.1 ->
+//     9.4, 16384 x 8192 at 2 39.8 -> 32.7, but 20480 x 5120 at 1 28.1 -> 31.3,
+//     16384 x 9216 at 2 32.4 -> 34.4, 16384 x 1024 at 1 7.6 -> 9.8.
+//   3-4 tokens: 4096 x 8192 12.3 -> 10.8, 16384 x 4096 19.9 -> 17.7, but 4096 x
+//     9216 13.7 -> 13.8, 16384 x 5120 21.4 -> 28.6, SwiGLU 12288 x 8192 26.9 -> 28.6.
+// At most 4 workgroups per CU: the lm_head's 7760 groups took 155 / 161 us at 1 /
+// 4 tokens with the quantizer launch and 156 / 163 this way. At 8 tokens, one row per
+// wave, merged q/k/v gained 1.0 us, gate+up 0.2, and down lost 3.4.
+inline bool fp8_quantizes_in_gemm(int64_t M, int64_t K, bool tiled, int cu_count, const DecodePlan& p) {
+  const int64_t cus = cu_count, steps = K / 128;
+  if (M > kDecodeQuantMaxRows || K > 16384 || p.splits != 1 || p.groups > 4 * cus) return false;
+  const int64_t bursts = ((steps + p.waves - 1) / p.waves + p.unroll - 1) / p.unroll;
+  const int64_t issued = bursts * p.unroll * p.waves;
+  const bool mostly_whole = 7 * issued <= 8 * steps;
+  const bool one_round = p.groups <= cus, one_burst = K >= 3072 && K <= 4096;
+  if (M <= 2) {
+    if (tiled) return K >= 2048 || M * p.rt * p.groups <= 4 * cus;
+    if (p.rt == 1) return one_round || K >= 2048;
+    return one_burst || (mostly_whole && (M == 1 || K <= 12288));
+  }
+  if (K > 12288) return false;
+  if (p.rt == 1 && one_round) return K >= 1024 && (tiled || K <= 4096 || mostly_whole);
+  if (!tiled) return one_burst || (mostly_whole && (p.rt == 1 || (one_round && K <= 8192)));
+  if (one_round) return K >= 2048;
+  if (p.rt == 1) return one_burst || K >= 6144;
+  return K >= 2048 && (K <= 4096 || (K <= 8192 && issued == steps));
 }
 hipError_t gemm_decode_quant(const uint16_t* x, int64_t ldx, const uint8_t* w, int64_t ldw, int M, int N, int K,
                              const DecodePlan& plan, const Epilogue& ep, hipStream_t stream);

@@ -12,7 +12,8 @@ kernels of ``libjeeves_fp8.so``, called through its C ABI:
 * the GEMM multiplies e4m3 by e4m3 on the FP8 MFMA units and applies
   ``acc * sx[m] * sw[n]`` (+ bias, + optional LoRA) in its epilogue;
 * 1-16 tokens run the HBM-bound split-K decode kernel, which quantizes 1-4
-  tokens itself on all but the widest weights; 17-128 tokens the
+  tokens itself where that is the faster (``jv_fp8_quantizes_in_gemm``); 17-128
+  tokens the
   batch-decode kernel on weights of up to one round of workgroups at
   K = 4096 / 12288 (whole k ranges of weights in registers, the batch's token
   tiles split across workgroups), else deep-ring 64x64 / 64x128 prefill tiles
@@ -42,7 +43,7 @@ from .fp8_weights import FP8, quantize_rows
 DECODE_MAX_ROWS = 64
 # Longest row the single-pass quantizer (and so the packed code layout) covers.
 QUANT_MAX_PACKED_COLS = 16384
-# Tokens up to which the decode GEMM quantizes its activations itself.
+# Tokens up to which the decode GEMM can quantize its activations itself.
 GEMM_QUANT_MAX_ROWS = 4
 BLOCK_K = 128
 TILE_COUNTER_SLOTS = 1 << 16
@@ -88,6 +89,12 @@ def _plan(device: torch.device, M: int, N: int, K: int, rank: int) -> tuple[int,
     if min(sizes[1:]) < 0:
         _lib.check(_lib.JV_ERR_HIP)
     return sizes
+
+
+@lru_cache(maxsize=4096)
+def _quantizes_in_gemm(device: torch.device, M: int, N: int, K: int, tiled: bool) -> bool:
+    """Whether ``fp8_matmul`` without LoRA of these sizes is one launch."""
+    return bool(_lib.lib().jv_fp8_quantizes_in_gemm(M, N, K, tiled, False, sm_count(device)))
 
 
 def _stream_counters(device: torch.device) -> torch.Tensor:
@@ -789,7 +796,8 @@ class FP8SwiGLU(nn.Module):
         packed = M > 0 and inter % BLOCK_K == 0 and inter <= QUANT_MAX_PACKED_COLS
         if self.gate_up.activations == "fp8" and self.fused():
             w, tiled = self.gate_up.kernel_weight()
-            if packed and lora_a is None and M <= GEMM_QUANT_MAX_ROWS:
+            if (packed and lora_a is None and M <= GEMM_QUANT_MAX_ROWS and x2.is_cuda
+                    and _quantizes_in_gemm(x2.device, M, self.down.out_features, inter, self.down.tiled)):
                 # A few tokens: the down GEMM quantizes h itself.
                 h = gate_up_swiglu(x2.to(torch.bfloat16), w, self.gate_up.scale, bias=self.gate_up.bias,
                                    lora=self.gate_up.lora, tiled=tiled)

@@ -252,3 +252,34 @@ def test_packed_layout_sizes_are_host_logic(product_lib):
 def test_hook_library_exports(hooks_lib):
     for name in ("th_encode", "th_encode_sweep", "th_quotient_sweep", "th_mfma32", "th_mfma16", "th_silu_sweep", "th_gemm_form"):
         assert hasattr(hooks_lib, name)
+
+
+# (tokens, N, K, tiled, SwiGLU, us with a quantizer launch, us in one launch),
+# on both sides of every line of the rule; graphs over 1 GiB of rotated weights
+ONE_OR_TWO_LAUNCHES = [
+    (1, 24576, 512, True, False, 7.2, 7.5), (1, 24576, 4096, True, False, 20.8, 18.4), (2, 20480, 1024, True, False, 8.9, 9.5),
+    (2, 20480, 2048, True, False, 12.3, 10.6), (4, 1024, 768, True, False, 4.37, 4.39), (4, 4096, 1536, True, False, 5.5, 4.9),
+    (4, 6144, 1024, True, False, 5.5, 5.9), (4, 6144, 2048, True, False, 7.1, 5.9), (4, 4096, 14336, True, False, 16.3, 17.0),
+    (4, 4096, 12288, True, False, 14.5, 14.1), (4, 24576, 4096, True, False, 21.0, 19.4),
+    (4, 24576, 12288, True, False, 56.1, 59.5), (4, 12288, 5120, True, False, 16.3, 16.7),
+    (4, 12288, 6144, True, False, 18.7, 18.3), (4, 32768, 8192, True, False, 55.6, 51.9),
+    (4, 24576, 5120, True, False, 25.6, 26.5), (3, 24576, 5120, True, False, 25.6, 26.5),
+    (1, 16384, 1024, False, False, 7.6, 9.8), (1, 8192, 4096, False, False, 12.1, 9.4), (1, 20480, 5120, False, False, 28.1, 31.3),
+    (1, 4096, 12288, False, False, 16.1, 13.1), (2, 16384, 8192, False, False, 39.8, 32.7),
+    (2, 16384, 9216, False, False, 32.4, 34.4), (4, 4096, 9216, False, False, 13.7, 13.8),
+    (4, 4096, 8192, False, False, 12.3, 10.8), (4, 16384, 5120, False, False, 21.4, 28.6),
+    (4, 16384, 4096, False, False, 19.9, 17.7), (1, 24576, 4096, True, True, 21.3, 19.5), (4, 24576, 4096, True, True, 21.4, 20.3),
+    (4, 8192, 1024, True, True, 6.0, 6.2), (4, 16384, 5120, True, True, 19.1, 21.8), (2, 24576, 768, True, True, 8.8, 9.8),
+    (2, 24576, 2048, False, True, 13.2, 15.1), (2, 24576, 4096, False, True, 26.0, 24.6),
+    (4, 12288, 8192, False, True, 26.9, 28.6),
+    (1, 248320, 4096, True, False, 155.0, 156.0), (4, 248320, 4096, True, False, 161.0, 163.0),
+]
+
+
+def test_decode_gemm_quantizes_where_that_is_faster(product_lib):
+    for M, N, K, tiled, swiglu, two, one in ONE_OR_TWO_LAUNCHES:
+        assert product_lib.jv_fp8_quantizes_in_gemm(M, N, K, tiled, swiglu, 256) == (one < two), (M, N, K, tiled, swiglu)
+    # never past 4 tokens, with a K split or past the packed quantizer's rows
+    assert not product_lib.jv_fp8_quantizes_in_gemm(5, 4096, 4096, True, False, 256)
+    assert not product_lib.jv_fp8_quantizes_in_gemm(1, 256, 4096, True, False, 256)
+    assert not product_lib.jv_fp8_quantizes_in_gemm(1, 4096, 16512, True, False, 256)

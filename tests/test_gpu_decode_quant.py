@@ -23,10 +23,12 @@ def same(a: torch.Tensor, b: torch.Tensor) -> bool:
 
 
 # 128 and 640: waves without steps and with one or two; 2560 and 4224: short
-# bursts; 16384: the longest row; 4112 and 70000 rows: more and far more than
-# one round of workgroups; 256: a K split, on the general path.
+# bursts; 16384: the longest row; 4112 rows up: two tiles per wave, with each
+# chunk count (4096 to 16384 columns); 256: a K split and 70000: far more than
+# one round of short rows, on the general path.
 @pytest.mark.parametrize("N,K", [(1024, 128), (1600, 640), (1040, 2560), (1024, 4096), (5000, 4096), (24576, 4096),
-                                 (4112, 4224), (4096, 12288), (1008, 16384), (70000, 512), (256, 4096)])
+                                 (4112, 4224), (4096, 12288), (1008, 16384), (70000, 512), (256, 4096), (16384, 1024),
+                                 (4112, 8192), (4112, 12288), (4112, 16384)])
 @pytest.mark.parametrize("M", [1, 2, 3, 4, 5])
 def test_quantizing_gemm_equals_quantizer_and_gemm(N, K, M):
     print(f"quantizing decode GEMM N={N} K={K} M={M}", flush=True)
