@@ -146,7 +146,7 @@ int jv_fp8_linear_noalloc(const void* x, int64_t ldx, const void* w, int64_t ldw
  * are. Arguments as jv_fp8_linear (no LoRA), but y must not overlap x; K a
  * positive multiple of 128.
  * workspace: jv_w8a16_workspace_bytes(M,N,K) bytes: the activations packed for
- * the decode kernel (17-64 tokens on large weights), then the split-K
+ * the decode kernel (17-64 tokens, where that is faster), then the split-K
  * partials of the decode kernel or of the prefill kernel's 64x64 tiles (0 for
  * most shapes). A workspace that holds the partials alone is taken too, the
  * activations then read as they are (same bits, slower). tile_counters as

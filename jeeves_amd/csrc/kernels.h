@@ -375,16 +375,44 @@ hipError_t w8a16_batch(const uint16_t* x, int64_t ldx, const uint8_t* w, int64_t
                        const BatchPlan& p, const float* sw, const uint16_t* bias, uint16_t* y, int64_t ldy,
                        hipStream_t stream);
 // Rows in the fragment order of w8a16_decode (packed_x there):
-// w8a16_packed_bytes(M, K) bytes. Packing is a launch of its own (2 us), so it
-// pays on large weights past 16 tokens and on all but small ones past 32 (us,
-// graphs over rotated weights, rows as they are vs packed: down M = 24 / 32 /
-// 64 22.6 / 26.6 / 47.6 vs 20.8 / 21.0 / 29.7, merged q/k/v 24 / 48 / 64 11.3 /
-// 16.6 / 20.6 vs 12.8 / 14.6 / 16.4, 5008 x 2560 32 / 48 / 64 8.6 / 11.2 / 13.5
-// vs 8.6 / 9.9 / 11.0; down at 16 tokens 17.3 vs 17.1). The wide weights whose
-// larger batches take prefill tiles (decode_kernel_for) and the batch-decode
-// plans stay without a workspace.
+// w8a16_packed_bytes(M, K) bytes. As rows, each workgroup's activation loads
+// take 64 line lookups per 1 KB, and the lookups grow with the rows in the
+// batch (a 16-token tile's rows past M repeat the last one and share its
+// lines); packed, they take 8 whatever M is, but the packing is a launch of its
+// own (2 us) and whole tiles are read. So packing pays by the rows in the last
+// tile, by K, and by how many workgroups each CU runs, half as much with two
+// weight tiles per activation load. The lines lie where 4200 timed pairs on
+// MI355X cross (17-64 tokens, 15 row lengths, 16 widths; rows as they are ->
+// packed, us, graphs over 1 GiB of rotated weights, N x K; kept, the packed side is
+// at most 6 % slower anywhere and 1.4 % off the faster side on average):
+//   17-32 tokens, several rounds: 10240 x 8192 at 17 / 24 33.2 / 40.3 -> 34.4 /
+//     34.4, 12288 x 2048 at 24 / 28 12.5 / 13.6 -> 12.9 / 12.9, two tiles per
+//     wave 16384 x 4096 at 20 / 24 19.7 / 20.9 -> 20.4 / 20.5, short rows 16384 x
+//     1024 at 32 8.2 -> 9.1; one round: 4096 x 12288 at 24 / 28 / 32 22.0 /
+//     24.2 / 26.4 -> 21.7 / 21.8 / 21.9, shorter rows 8192 x 8192 at 32 22.4 -> 23.8.
+//   33-48 tokens, one tile per wave: 4096 x 8192 at 33 20.4 -> 19.3, 4096 x
+//     3072 at 33 / 40 9.5 / 10.5 -> 10.6 / 10.5, 4096 x 1024 at 48 5.7 -> 6.1,
+//     several rounds 12288 x 1024 at 33 10.5 -> 9.9; two tiles: 6144 x 12288 at
+//     33 / 36 32.6 / 34.2 -> 33.2 / 33.2, 6144 x 4096 at 36 / 44 13.7 / 15.3 ->
+//     14.2 / 14.3, several rounds 16384 x 4096 at 33 / 36 25.2 / 26.6 -> 25.6 /
+//     25.6, 16384 x 1024 at 36 9.3 -> 10.2.
+//   49-64 tokens: 4096 x 2048 at 64 10.3 -> 8.4, 16384 x 2048 22.9 -> 19.8, two
+//     tiles 6144 x 2560 at 49 12.8 -> 12.2, 8192 x 2048 at 49 11.0 -> 12.3.
+// The wide weights whose larger batches take prefill tiles (decode_kernel_for)
+// and the batch-decode plans stay without a workspace.
 inline bool w8a16_packs(int64_t M, int64_t N, int64_t K, int cu_count) {
-  return M > 16 && 2 * ((N + 63) / 64) < 3 * (int64_t)cu_count && N * K >= (M > 32 ? int64_t(8) << 20 : int64_t(48) << 20);
+  if (M <= 16 || M > kDecodeMaxRows || 2 * ((N + 63) / 64) >= 3 * (int64_t)cu_count) return false;
+  const DecodePlan p = decode_plan(M, N, K, cu_count);
+  const bool one_round = p.groups <= cu_count;
+  if (M <= 32) {
+    if (one_round) return K >= 10240 && M >= 28;
+    return K >= 2048 && M >= (p.rt == 2 ? 24 : K >= 3072 ? 22 : 28);
+  }
+  if (M <= 48) {
+    if (p.rt == 1) return one_round ? K >= 2048 && M >= (K >= 5120 ? 33 : 40) : K >= 1024;
+    return one_round ? K >= 4096 && M >= (K >= 10240 ? 36 : 44) : K >= 2048 && M >= 36;
+  }
+  return one_round ? K >= (p.rt == 1 ? 2048 : 2560) : p.rt == 2 || K >= 1024;
 }
 inline int64_t w8a16_packed_bytes(int64_t M, int64_t K) { return (M + 15) / 16 * 16 * K * 2; }
 hipError_t w8a16_pack_x(const uint16_t* x, int64_t ldx, int M, int K, uint16_t* out, hipStream_t stream);
