@@ -47,10 +47,12 @@ QUANT_MAX_PACKED_COLS = 16384
 GEMM_QUANT_MAX_ROWS = 4
 BLOCK_K = 128
 TILE_COUNTER_SLOTS = 1 << 16
-# One row count per kernel variant: 1-4 decode token tiles, then prefill
-# batches that select the 256x256, 256x128, 128x128, 64x128 and 64x64 tiles on
-# large and small N (inference/fp8.py:32 plays the same role for Triton's JIT).
-WARM_ROWS = (1, 16, 17, 32, 33, 48, 49, 64, 65, 256, 300, 2048)
+# One row count per kernel variant: the decode GEMM quantizing for itself (1, 2
+# and 3-4 tokens), 1-4 decode token tiles, each full and with one row (the
+# W8A16 mode packs the activations of full ones), then prefill batches that
+# select the 256x256, 256x128, 128x128, 64x128 and 64x64 tiles on large and
+# small N (inference/fp8.py:32 plays the same role for Triton's JIT).
+WARM_ROWS = (1, 2, 4, 16, 17, 32, 33, 48, 49, 64, 65, 256, 300, 2048)
 LORA_RANKS = (16,)
 
 TILE_COUNTERS: dict[tuple[torch.device, int], torch.Tensor] = {}

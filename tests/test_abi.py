@@ -283,3 +283,21 @@ def test_decode_gemm_quantizes_where_that_is_faster(product_lib):
     assert not product_lib.jv_fp8_quantizes_in_gemm(5, 4096, 4096, True, False, 256)
     assert not product_lib.jv_fp8_quantizes_in_gemm(1, 256, 4096, True, False, 256)
     assert not product_lib.jv_fp8_quantizes_in_gemm(1, 4096, 16512, True, False, 256)
+
+
+def test_warm_rows_reach_every_decode_kernel(product_lib):
+    """Each kernel that a batch of 1-64 tokens of some weight selects is run by
+    one of warm()'s row counts on that weight."""
+    from jeeves_amd.fp8 import WARM_ROWS
+
+    def kernel(M, N, K, tiled):
+        if product_lib.jv_fp8_quantizes_in_gemm(M, N, K, tiled, False, 256):
+            return "quantizing", {1: 1, 2: 2, 3: 4, 4: 4}[M]
+        kind = tuple(launch_shape(product_lib, M, N, K))
+        return kind[0], (M + 15) // 16 if kind[0] == 0 else kind[1:]
+
+    for N, K in ((1024, 4096), (4096, 4096), (6144, 4096), (24576, 4096), (4096, 12288), (2560, 2560), (8192, 1024), (256, 4096)):
+        for tiled in (True, False):
+            warmed = {kernel(M, N, K, tiled) for M in WARM_ROWS}
+            for M in range(1, 65):
+                assert kernel(M, N, K, tiled) in warmed, (M, N, K, tiled)
