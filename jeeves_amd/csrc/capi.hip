@@ -336,8 +336,8 @@ int jv_fp8_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, const 
                                               (int)lora_rank, lora_t, packed, s),
                           "activation quantization launch"))
     return rc;
-  return run_gemm(codes, packed ? 0 : K, packed, sx, (const uint8_t*)w, ldw, w_scale, (const uint16_t*)bias, lora_t, (const uint16_t*)lora_b,
-                  lora_rank, lora_scaling, (uint16_t*)y, ldy, M, N, K, ws, rest, tile_counters, n_counters, s);
+  return run_gemm(codes, packed ? 0 : K, packed, sx, (const uint8_t*)w, ldw, w_scale, (const uint16_t*)bias, lora_t,
+                  (const uint16_t*)lora_b, lora_rank, lora_scaling, (uint16_t*)y, ldy, M, N, K, ws, rest, tile_counters, n_counters, s);
 }
 
 int64_t jv_w8a16_workspace_bytes(int64_t M, int64_t N, int64_t K) {
@@ -410,8 +410,8 @@ int jv_w8a16_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, cons
                   (long long)need);
     partial = reinterpret_cast<float*>(workspace);
   }
-  return hip_status(jv::w8a16_decode((const uint16_t*)x, ldx, packed_x, (const uint8_t*)w, ldw, (int)M, (int)N, (int)K, plan, partial,
-                                     tile_counters, w_scale, (const uint16_t*)bias, (uint16_t*)y, ldy, s),
+  return hip_status(jv::w8a16_decode((const uint16_t*)x, ldx, packed_x, (const uint8_t*)w, ldw, (int)M, (int)N, (int)K, plan,
+                                     partial, tile_counters, w_scale, (const uint16_t*)bias, (uint16_t*)y, ldy, s),
                     "W8A16 decode GEMM launch");
 }
 

@@ -229,12 +229,6 @@ __device__ __forceinline__ uint32_t row16_max_u32_in_lane15(uint32_t v) {
   return v;
 }
 
-__device__ __forceinline__ float wave_sum_f32(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-
 // Max of two packed 16-bit magnitudes (v_pk_max_u16).
 __device__ __forceinline__ uint32_t pk_max_u16(uint32_t a, uint32_t b) {
   u16x2 va = __builtin_bit_cast(u16x2, a);

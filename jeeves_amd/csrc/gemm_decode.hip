@@ -42,13 +42,14 @@ constexpr int kMaxDecodeSplits = 16;
 // at M = 16 on gate+up (19.7 vs 18.7 us), even at one split.
 // MQ > 0: the workgroup quantizes the activations itself (1 to MQ tokens, MT
 // = 1): xq is then the bf16 rows (ldxq their stride in elements), and NCQ
-// 8-element chunks per lane cover a row shared by WAVES / MQ waves. The row maxima, scales and codes
-// are quant_row's, bit for bit. The rows' loads go out first, the first burst
-// of weights right behind them, so the quantization runs while the weights are
-// on their way; the codes go to LDS, M rows of them, where the packed codes in
-// memory come in whole 16-row tiles (64 KB of L2 reads per workgroup at K =
-// 4096, as much as its weights). A linear saves the quantizer's launch and a
-// dependent kernel boundary: fp8_quantizes_in_gemm (kernels.h) has the times.
+// 8-element chunks per lane cover a row shared by WAVES / MQ waves. The row
+// maxima, scales and codes are quant_row's, bit for bit. The rows' loads go out
+// first, the first burst of weights right behind them, so the quantization runs
+// while the weights are on their way; the codes go to LDS, M rows of them, where
+// the packed codes in memory come in whole 16-row tiles (64 KB of L2 reads per
+// workgroup at K = 4096, as much as its weights). A linear saves the quantizer's
+// launch and a dependent kernel boundary: fp8_quantizes_in_gemm (kernels.h) has
+// the times, and the sizes.
 template <int MT, int RT, int WAVES, int UNROLL, bool PACKX, int RANK, bool PACKW, bool SW = false, bool SPLIT = false,
           int MQ = 0, int NCQ = 1>
 __global__ __launch_bounds__(64 * WAVES) void gemm_decode_kernel(const uint8_t* __restrict__ xq, int64_t ldxq,
@@ -114,7 +115,9 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_decode_kernel(const uint8_t* 
   const uint8_t* xp[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
-    xp[mt] = MQ > 0 ? nullptr : PACKX ? xq + (int64_t)mt * ksteps * 2048 + lane * 16 : xq + (int64_t)min(mt * 16 + li, M - 1) * ldxq + lk;
+    xp[mt] = MQ > 0  ? nullptr
+             : PACKX ? xq + (int64_t)mt * ksteps * 2048 + lane * 16
+                     : xq + (int64_t)min(mt * 16 + li, M - 1) * ldxq + lk;
 
   // Each thread's outputs (idx = threadIdx.x + j * 64 WAVES; channel fastest)
   // and their scales and bias, loaded before the weight stream so the
@@ -152,22 +155,16 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_decode_kernel(const uint8_t* 
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[rt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // One burst of up to UNROLL k steps: all its loads are issued, then the
-  // MFMAs consume them. A full burst is straight-line code, so each step's
-  // MFMAs wait only for that step's data; the last, partial burst guards each
-  // step with a scalar branch (s and s_end are wave-uniform).
-  // The burst's addresses are one base per operand plus constant offsets
-  // (u steps of 2 KB packed or 128 B row-major), which the loads take as
-  // immediates instead of a 64-bit add per step (0.5 us of the 1 us above).
   // Codes of the quantizing form in LDS, one row every K + kCodePad bytes (the
   // pad puts the rows of a 16-lane read in different banks).
   constexpr int kCodePad = 32;
   extern __shared__ __attribute__((aligned(16))) uint8_t qcodes[];
   const uint8_t* ql = qcodes + (int64_t)(li % QR) * (K + kCodePad) + lk;
   i32x4 wa[UNROLL][RT][2];
-  // A short burst repeats its last step, so the loads are unconditional and
-  // the wait for the rows does not take the weights in.
-  // Tiled weights: a wave-uniform base per tile and step, one lane offset.
+  // The quantizing form's burst of weights. A short one repeats its last step,
+  // so the loads are unconditional and the wait for the rows does not take the
+  // weights in. Tiled weights: a wave-uniform base per tile and step, one lane
+  // offset.
   auto load_w = [&](int s) {
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
@@ -195,6 +192,13 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_decode_kernel(const uint8_t* 
       for (int rt = 0; rt < RT; ++rt) acc[rt][0] = mfma_16x16x128_fp8(cat8(wa[u][rt][0], wa[u][rt][1]), b, acc[rt][0]);
     }
   };
+  // One burst of up to UNROLL k steps: all its loads are issued, then the
+  // MFMAs consume them. A full burst is straight-line code, so each step's
+  // MFMAs wait only for that step's data; the last, partial burst guards each
+  // step with a scalar branch (s and s_end are wave-uniform).
+  // The burst's addresses are one base per operand plus constant offsets
+  // (u steps of 2 KB packed or 128 B row-major), which the loads take as
+  // immediates instead of a 64-bit add per step (0.5 us of the 1 us above).
   auto burst = [&](int s, auto full) {
     constexpr bool FULL = decltype(full)::value;
     constexpr int WSTEP = PACKW ? 2048 : 128, XSTEP = PACKX ? 2048 : 128;
@@ -505,17 +509,25 @@ static hipError_t launch_decode_quant(const uint16_t* x, int64_t ldx, const uint
   return hipGetLastError();
 }
 
-// NC: 8-element chunks of a row per thread of the workgroup.
+// NC: 8-element chunks of a row per thread of the workgroup. Only the instances
+// that fp8_quantizes_in_gemm takes: at 3-4 tokens rows of at most 12288 elements
+// (NC 3 of 8 waves), and with four waves of two tiles (rows below 2048) 1-2
+// tokens on tiled weights.
 template <int RT, int W, int NC, bool SW>
 static hipError_t launch_decode_quant_m(const uint16_t* x, int64_t ldx, const uint8_t* w, int64_t ldw, int M, int N, int K,
                                         const DecodePlan& p, const Epilogue& ep, hipStream_t stream) {
+  constexpr bool kShort = RT == 2 && W == 4;
 #define JV_DECODE_QUANT(MQ)                                                                                       \
-  return ldw == 0 ? launch_decode_quant<RT, W, NC * MQ, MQ, true, SW>(x, ldx, w, ldw, M, N, K, p, ep, stream)      \
-                  : launch_decode_quant<RT, W, NC * MQ, MQ, false, SW>(x, ldx, w, ldw, M, N, K, p, ep, stream)
+  {                                                                                                                \
+    if (ldw == 0) return launch_decode_quant<RT, W, NC * MQ, MQ, true, SW>(x, ldx, w, ldw, M, N, K, p, ep, stream); \
+    if constexpr (!kShort) return launch_decode_quant<RT, W, NC * MQ, MQ, false, SW>(x, ldx, w, ldw, M, N, K, p, ep, stream); \
+  }
   if (M == 1) JV_DECODE_QUANT(1);
   if (M == 2) JV_DECODE_QUANT(2);
-  JV_DECODE_QUANT(4);
+  if constexpr (NC <= 3 && !kShort)
+    if (M > 2) JV_DECODE_QUANT(4);
 #undef JV_DECODE_QUANT
+  return hipErrorInvalidValue;
 }
 
 hipError_t gemm_decode_quant(const uint16_t* x, int64_t ldx, const uint8_t* w, int64_t ldw, int M, int N, int K,
@@ -531,10 +543,10 @@ hipError_t gemm_decode_quant(const uint16_t* x, int64_t ldx, const uint8_t* w, i
       if (ep.half) return launch_decode_quant_m<RT_, W_, NC_, true>(x, ldx, w, ldw, M, N, K, p, ep, stream);     \
     return launch_decode_quant_m<RT_, W_, NC_, false>(x, ldx, w, ldw, M, N, K, p, ep, stream);                   \
   }
-  // decode_plan takes 4 waves up to K = 4096 (two chunks per thread), 8 above.
+  // decode_plan takes four waves up to K = 4096 with one tile per wave and below
+  // 2048 with two, eight above.
   JV_DECODE_QUANT_CASE(1, 4, 2)
-  JV_DECODE_QUANT_CASE(2, 4, 2)
-  JV_DECODE_QUANT_CASE(1, 8, 1)
+  JV_DECODE_QUANT_CASE(2, 4, 1)
   JV_DECODE_QUANT_CASE(2, 8, 1)
   JV_DECODE_QUANT_CASE(1, 8, 2)
   JV_DECODE_QUANT_CASE(2, 8, 2)

@@ -279,6 +279,16 @@ ONE_OR_TWO_LAUNCHES = [
 def test_decode_gemm_quantizes_where_that_is_faster(product_lib):
     for M, N, K, tiled, swiglu, two, one in ONE_OR_TWO_LAUNCHES:
         assert product_lib.jv_fp8_quantizes_in_gemm(M, N, K, tiled, swiglu, 256) == (one < two), (M, N, K, tiled, swiglu)
+    # only where the kernel has an instance: at 3-4 tokens rows up to 12288, and
+    # with two tiles per wave on rows below 2048 tiled weights at 1-2 tokens
+    for K in range(128, 16384 + 128, 128):
+        for N in (512, 4096, 4112, 8192, 8208, 16352, 16384, 24576, 32768, 65536):
+            for tiled in (True, False):
+                for swiglu in (True, False):
+                    assert not (K > 12288 and product_lib.jv_fp8_quantizes_in_gemm(4, N, K, tiled, swiglu, 256))
+                    if K < 2048 and (swiglu or N > 16368):
+                        assert not product_lib.jv_fp8_quantizes_in_gemm(4, N, K, tiled, swiglu, 256)
+                        assert tiled or not product_lib.jv_fp8_quantizes_in_gemm(1, N, K, tiled, swiglu, 256)
     # never past 4 tokens, with a K split or past the packed quantizer's rows
     assert not product_lib.jv_fp8_quantizes_in_gemm(5, 4096, 4096, True, False, 256)
     assert not product_lib.jv_fp8_quantizes_in_gemm(1, 256, 4096, True, False, 256)
