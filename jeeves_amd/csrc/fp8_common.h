@@ -236,6 +236,14 @@ __device__ __forceinline__ uint32_t pk_max_u16(uint32_t a, uint32_t b) {
   return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(va, vb));
 }
 
+// The maximum am joined by the magnitudes of a chunk of 8 bf16 elements.
+__device__ __forceinline__ uint32_t pk_max_chunk(uint32_t am, uint4 v) {
+  am = pk_max_u16(am, v.x & 0x7FFF7FFFu);
+  am = pk_max_u16(am, v.y & 0x7FFF7FFFu);
+  am = pk_max_u16(am, v.z & 0x7FFF7FFFu);
+  return pk_max_u16(am, v.w & 0x7FFF7FFFu);
+}
+
 // ---------------------------------------------------------------------------
 // MFMA wrappers. Format code 0 selects FP8 E4M3 for both operands; zero scale
 // operands select the unscaled v_mfma_f32_{32x32x64,16x16x128}_f8f6f4.

@@ -246,10 +246,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_decode_kernel(const uint8_t* 
     // a repeated last chunk does not change the maximum
 #pragma unroll
     for (int i = 0; i < NCQ; ++i) {
-      am = pk_max_u16(am, xr[i].x & 0x7FFF7FFFu);
-      am = pk_max_u16(am, xr[i].y & 0x7FFF7FFFu);
-      am = pk_max_u16(am, xr[i].z & 0x7FFF7FFFu);
-      am = pk_max_u16(am, xr[i].w & 0x7FFF7FFFu);
+      am = pk_max_chunk(am, xr[i]);
     }
     am = wave_max_u32(max(am & 0xFFFFu, am >> 16));
     if constexpr (QW > 1) {

@@ -43,10 +43,7 @@ struct Unit<uint16_t> {
     uint32_t am = 0;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      am = pk_max_u16(am, v[i].x & 0x7FFF7FFFu);
-      am = pk_max_u16(am, v[i].y & 0x7FFF7FFFu);
-      am = pk_max_u16(am, v[i].z & 0x7FFF7FFFu);
-      am = pk_max_u16(am, v[i].w & 0x7FFF7FFFu);
+      am = pk_max_chunk(am, v[i]);
     }
     return max(am & 0xFFFFu, am >> 16);
   }

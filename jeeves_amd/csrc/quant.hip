@@ -24,17 +24,6 @@ __device__ __forceinline__ uint32_t block_max(uint32_t v, uint32_t* red) {
   return v;
 }
 
-// Packed codes of more than one 16-token tile: the 16 rows of a tile are
-// quantized on one XCD (the hardware hands consecutive workgroups to the 8
-// XCDs in turn), so the 16-byte pieces they write into each fragment meet in
-// one L2 and reach memory as whole lines. Workgroup b serves row 16 t + j % 16
-// of tile t = b % 8 + 8 (j / 16), j = b / 8; -1 past the last tile.
-__device__ __forceinline__ int packed_tile_row(int b, int tiles) {
-  const int j = b >> 3;
-  const int t = (b & 7) + 8 * (j >> 4);
-  return t < tiles ? t * 16 + (j & 15) : -1;
-}
-
 // NC chunks of 8 elements per thread kept in registers (K <= NC * 8 * THREADS).
 // XCD_ROWS: workgroups map to rows through packed_tile_row.
 template <int THREADS, int NC, bool SWIGLU, int RANK, bool PACKED, bool XCD_ROWS = false>
@@ -99,10 +88,7 @@ __global__ __launch_bounds__(kQuantThreads) void quant_rows_bf16_long_kernel(con
   uint32_t am = 0;
   for (int c = threadIdx.x; c < nchunks; c += kQuantThreads) {
     const uint4 v = *reinterpret_cast<const uint4*>(xr + (int64_t)c * 8);
-    am = pk_max_u16(am, v.x & 0x7FFF7FFFu);
-    am = pk_max_u16(am, v.y & 0x7FFF7FFFu);
-    am = pk_max_u16(am, v.z & 0x7FFF7FFFu);
-    am = pk_max_u16(am, v.w & 0x7FFF7FFFu);
+    am = pk_max_chunk(am, v);
   }
   am = max(am & 0xFFFFu, am >> 16);
   const uint32_t amax_bits = block_max(am, red);

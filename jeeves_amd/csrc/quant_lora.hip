@@ -33,12 +33,8 @@ __global__ __launch_bounds__(kThreads) void quant_lora_kernel(const uint16_t* __
   __shared__ float red_t[ROWS][NW][kRank];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nchunks = K >> 3;
-  // The workgroups of a 16-row tile run on one XCD (consecutive workgroups go
-  // to the 8 XCDs in turn), so the pieces they write into each fragment meet
-  // in one L2.
-  const int j = blockIdx.x >> 3;
-  const int row0 = ((int)(blockIdx.x & 7) + 8 * (j / (16 / ROWS))) * 16 + (j % (16 / ROWS)) * ROWS;
-  if (row0 >= (PACKED ? (M + 15) / 16 * 16 : M)) return;  // the whole workgroup
+  const int row0 = packed_tile_row<ROWS>((int)blockIdx.x, (M + 15) >> 4);
+  if (row0 < 0 || (!PACKED && row0 >= M)) return;  // the whole workgroup
 
   uint4 v[ROWS][NC];
 #pragma unroll
@@ -79,10 +75,7 @@ __global__ __launch_bounds__(kThreads) void quant_lora_kernel(const uint16_t* __
     // A repeated last chunk does not change the maximum.
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
-      am = pk_max_u16(am, v[r][i].x & 0x7FFF7FFFu);
-      am = pk_max_u16(am, v[r][i].y & 0x7FFF7FFFu);
-      am = pk_max_u16(am, v[r][i].z & 0x7FFF7FFFu);
-      am = pk_max_u16(am, v[r][i].w & 0x7FFF7FFFu);
+      am = pk_max_chunk(am, v[r][i]);
     }
     am = wave_max_u32(max(am & 0xFFFFu, am >> 16));
     if (lane == 0) red_max[r][wave] = am;

@@ -76,6 +76,20 @@ __device__ __forceinline__ float lora_wave_sum(float (&t)[RANK], int lane) {
   return t[0] + __shfl_xor(t[0], 32, 64);
 }
 
+// Packed codes of more than one 16-token tile: the workgroups of a tile run on
+// one XCD (the hardware hands consecutive workgroups to the 8 XCDs in turn), so
+// the pieces they write into each fragment meet in one L2 and reach memory as
+// whole lines. Workgroup b of ROWS rows each serves the rows from 16 t + ROWS
+// (j % (16 / ROWS)) of tile t = b % 8 + 8 (j / (16 / ROWS)), j = b / 8; -1 past
+// the last tile.
+template <int ROWS = 1>
+__device__ __forceinline__ int packed_tile_row(int b, int tiles) {
+  constexpr int per_tile = 16 / ROWS, shift = __builtin_ctz(per_tile);
+  const int j = b >> 3;
+  const int t = (b & 7) + 8 * (j >> shift);
+  return t < tiles ? t * 16 + (j & (per_tile - 1)) * ROWS : -1;
+}
+
 // LDS the quantizer needs: one word per wave for the row maximum and, with
 // LoRA, RANK partial sums per wave.
 template <int THREADS, int RANK>
@@ -127,10 +141,7 @@ __device__ __forceinline__ void quant_row(int row, const uint16_t* __restrict__ 
     } else {
       v[i] = uint4{0, 0, 0, 0};
     }
-    am = pk_max_u16(am, v[i].x & 0x7FFF7FFFu);
-    am = pk_max_u16(am, v[i].y & 0x7FFF7FFFu);
-    am = pk_max_u16(am, v[i].z & 0x7FFF7FFFu);
-    am = pk_max_u16(am, v[i].w & 0x7FFF7FFFu);
+    am = pk_max_chunk(am, v[i]);
   }
   if constexpr (RANK > 0) {
     // A's chunks are loaded 8 ranks at a time, the next batch while this
