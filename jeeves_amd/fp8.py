@@ -515,6 +515,13 @@ def quantize_swiglu_output(h: torch.Tensor, amax: torch.Tensor | None = None, *,
     return out + (t,) if rank else out
 
 
+def _weight_key(weight: torch.Tensor) -> tuple[int, int]:
+    """What a tiled copy of ``weight`` remembers it by. Inference tensors (made
+    under torch.inference_mode) keep no version counter: their key is the
+    address alone, and in-place writes to them need retile()."""
+    return weight.data_ptr(), (-1 if weight.is_inference() else weight._version)
+
+
 class FP8Linear(nn.Module):
     """``inference/fp8.py:151-185``: buffers ``weight`` (float8_e4m3fn [N,K],
     row-major, as the reference keeps it) and ``scale`` (float32 [N]),
@@ -561,20 +568,6 @@ class FP8Linear(nn.Module):
         if module.weight.device.type == "cuda":
             module.kernel_weight()
 
-    def _tensor(self, name: str) -> torch.Tensor:
-        """``self.<name>``, past ``Module.__getattr__`` (0.5 us against 0.1, four
-        times a call) while it is the registered buffer; a ``Parameter`` in its
-        place, a parametrization or a plain attribute is no buffer."""
-        t = self._buffers.get(name)
-        return getattr(self, name) if t is None else t
-
-    def _weight_key(self) -> tuple[int, int]:
-        # Inference tensors (made under torch.inference_mode) keep no version
-        # counter: their key is the address alone, and in-place writes to them
-        # need retile().
-        w = self._tensor("weight")
-        return w.data_ptr(), (-1 if torch.is_inference(w) else w._version)
-
     def kernel_weight(self) -> tuple[torch.Tensor, bool]:
         """The codes the kernels read and whether they are tiled: the tiled
         copy, rebuilt first if ``weight`` changed since it was made, or
@@ -582,13 +575,23 @@ class FP8Linear(nn.Module):
         write that bumps its version counter (``copy_``, ``load_state_dict``);
         writes that bypass the counter (through ``weight.data``, or into an
         inference tensor) must be followed by ``retile()``."""
+        # Buffers are read past Module.__getattr__ (0.5 us against 0.1, four times
+        # a call); a Parameter in a buffer's place, a parametrization or a plain
+        # attribute is none.
+        buffers = self._buffers
+        w = buffers.get("weight")
+        if w is None:
+            w = self.weight
         if not self.tiled:
-            return self._tensor("weight"), False
-        key = self._weight_key()
+            return w, False
+        codes = buffers.get("tiled_codes")
+        if codes is None:
+            codes = self.tiled_codes
+        key = _weight_key(w)
         if self._tiled_from != key:
-            _tile_into(self._tensor("weight"), self._tensor("tiled_codes"))
+            _tile_into(w, codes)
             self._tiled_from = key
-        return self._tensor("tiled_codes"), True
+        return codes, True
 
     @torch.no_grad()
     def retile(self) -> None:
@@ -634,39 +637,37 @@ class FP8Linear(nn.Module):
         parametrization, say), inference tensors outside inference mode, which
         ``copy_`` refuses to write, and a weight whose memory the kernel's own
         writes would change, or that torch negates on reading."""
-        codes, scale = self._buffers.get("weight"), self._buffers.get("scale")
-        tiled = self._buffers.get("tiled_codes") if self.tiled else None
-        if codes is None or scale is None or (self.tiled and tiled is None):
+        buffers = self._buffers
+        codes, scale = buffers.get("weight"), buffers.get("scale")
+        tiled = buffers.get("tiled_codes") if self.tiled else None
+        if (codes is None or scale is None or (self.tiled and tiled is None) or weight.layout != torch.strided
+                or weight.dim() != 2 or getattr(self.load_codes, "__func__", None) is not FP8Linear.load_codes):
             return False
-        N, K = codes.shape
-        dev = codes.device
-        if (getattr(self.load_codes, "__func__", None) is not FP8Linear.load_codes or dev.type != "cuda" or weight.is_neg()
-                or weight.dtype not in (torch.bfloat16, torch.float32) or weight.shape != codes.shape
-                or not N or not K or K % 16 or K > QUANT_MAX_PACKED_COLS or codes.dtype != FP8
-                or scale.dtype != torch.float32 or scale.shape != (N,) or not scale.is_contiguous() or scale.device != dev
-                or weight.layout != torch.strided or not _rows_aligned(weight, weight.element_size()) or weight.stride(0) < K
-                or not codes.is_contiguous() or codes.data_ptr() % 16):
+        N, K = shape = codes.shape
+        dev, elem, stride = codes.device, weight.element_size(), weight.stride(0)
+        src, dst, dst_scale = weight.data_ptr(), codes.data_ptr(), scale.data_ptr()
+        dst_tiled = None if tiled is None else tiled.data_ptr()
+        if (dev.type != "cuda" or weight.dtype not in (torch.bfloat16, torch.float32) or weight.shape != shape or weight.is_neg()
+                or not N or not K or K % 16 or K > QUANT_MAX_PACKED_COLS or codes.dtype != FP8 or not codes.is_contiguous()
+                or weight.stride(1) != 1 or stride < K or (stride * elem) % 16 or src % 16 or dst % 16
+                or scale.dtype != torch.float32 or scale.shape != (N,) or not scale.is_contiguous() or scale.device != dev):
             return False
-        if tiled is not None and (tiled.device != dev or tiled.shape != codes.shape or tiled.element_size() != 1
-                                  or not tiled.is_contiguous() or tiled.data_ptr() % 16):
+        if tiled is not None and (tiled.device != dev or tiled.shape != shape or tiled.element_size() != 1
+                                  or not tiled.is_contiguous() or dst_tiled % 16):
             return False
-        if not torch.is_inference_mode_enabled() and (torch.is_inference(codes) or torch.is_inference(scale)):
+        if (codes.is_inference() or scale.is_inference()) and not torch.is_inference_mode_enabled():
             return False
-        first, last = weight.data_ptr(), weight.data_ptr() + ((N - 1) * weight.stride(0) + K) * weight.element_size()
-        if any(t.data_ptr() < last and first < t.data_ptr() + t.numel() * t.element_size()
-               for t in (codes, scale, tiled) if t is not None):
+        end = src + ((N - 1) * stride + K) * elem
+        if (dst < end and src < dst + N * K or dst_scale < end and src < dst_scale + 4 * N
+                or dst_tiled is not None and dst_tiled < end and src < dst_tiled + N * K):
             return False
         with _device_guard(dev):
-            _lib.check(_lib.lib().jv_fp8_load_weight(weight.data_ptr(), weight.stride(0), weight.element_size(), N, K,
-                                                     codes.data_ptr(), K, scale.data_ptr(),
-                                                     tiled.data_ptr() if tiled is not None else None, _stream(dev)))
+            _lib.check(_lib.lib().jv_fp8_load_weight(src, stride, elem, N, K, dst, K, dst_scale, dst_tiled, _stream(dev)))
         # The kernel's writes count as in-place ones, so that a merged module
-        # over these buffers sees them.
-        for t in (codes, scale):
-            if not torch.is_inference(t):
-                torch.autograd.graph.increment_version(t)
+        # over these buffers sees them (inference tensors count none).
+        torch.autograd.graph.increment_version((codes, scale))
         if tiled is not None:
-            self._tiled_from = self._weight_key()
+            self._tiled_from = _weight_key(codes)
         return True
 
     def set_lora(self, a: torch.Tensor, b: torch.Tensor, scaling: float) -> None:
@@ -690,11 +691,11 @@ class FP8Linear(nn.Module):
         merged.weight, merged.scale = torch.cat([p.weight for p in parts]), torch.cat([p.scale for p in parts])
         merged.tiled = tiled
         merged.tiled_codes = torch.cat(copies) if tiled else None
-        merged._tiled_from = merged._weight_key() if tiled else None
+        merged._tiled_from = _weight_key(merged.weight) if tiled else None
         tiles = merged.tiled_codes.split(sizes) if tiled else [None] * len(parts)
         for p, weight, scale, t in zip(parts, merged.weight.split(sizes), merged.scale.split(sizes), tiles):
             p.weight, p.scale, p.tiled, p.tiled_codes = weight, scale, tiled, t
-            p._tiled_from = p._weight_key() if tiled else None
+            p._tiled_from = _weight_key(p.weight) if tiled else None
         return merged
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
@@ -705,7 +706,9 @@ class FP8Linear(nn.Module):
         if x2.stride(-1) != 1:
             x2 = x2.contiguous()
         w, tiled = self.kernel_weight()
-        scale = self._tensor("scale")
+        scale = self._buffers.get("scale")
+        if scale is None:
+            scale = self.scale
         if self.activations == "bf16":
             y = fp8_matmul_w8a16(x2, w, scale, bias=self.bias, tiled=tiled)
         else:
