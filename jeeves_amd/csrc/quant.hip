@@ -228,9 +228,12 @@ hipError_t quant_rows_bf16(const uint16_t* x, int64_t ldx, int64_t M, int K, uin
                            const uint16_t* lora_a, int rank, float* lora_t, bool packed, hipStream_t stream) {
   if (M == 0) return hipSuccess;
   const int nc = quant_chunks(K);
-  // Two rows per workgroup once the launch fills the CUs with them (the line
-  // lies between 256 and 512 rows at K = 12288: 10.1 vs 11.7 and 15.8 vs 14.5
-  // us, between 512 and 1024 at K = 4096: 6.6 vs 6.8 and 10.6 vs 9.3).
+  // Two rows per workgroup once the launch fills the CUs with them: between 256
+  // and 512 rows above K = 4096 (one row -> two, us: 10.1 -> 11.7 at 256 rows of
+  // 12288; at 512 rows of 4224 / 5120 / 8192 / 12288 / 16384 8.5 / 8.4 / 9.7 /
+  // 13.4 / 17.5 -> 7.8 / 7.9 / 9.3 / 12.4 / 15.7), between 512 and 1024 up to it
+  // (4096: 6.6 -> 6.8 at 512, 9.4 -> 8.3 at 1024; 2048: 6.2 -> 5.6 at 1024, 1024: 4.9
+  // -> 5.2, and 6.0 -> 5.7 at 1536).
   if (rank == 16 && nc != 0 && (M >= 1024 || (M >= 512 && K > 4096)))
     return quant_lora_bf16(x, ldx, M, K, codes, ldc, scales, lora_a, lora_t, packed, stream);
   if (packed) {
