@@ -306,8 +306,8 @@ constexpr int kDecodeQuantMaxRows = 4;
 // us, graphs over 1 GiB of rotated weights, N x K; 3 tokens run the kernel of
 // 4). Tiled weights:
 //   1-2 tokens: 24576 x 4096 at 1 20.8 -> 18.4, 20480 x 2048 at 2 12.3 -> 10.6;
-//     below K = 2048 up to 4 CUs' worth of tiles per token: 20480 x 1024 at 2
-//     8.9 -> 9.5, 24576 x 512 at 1 7.2 -> 7.5.
+//     below K = 2048 while tokens x 16-row tiles is at most 4 per CU: past that
+//     20480 x 1024 at 2 8.9 -> 9.5, 24576 x 512 at 1 7.2 -> 7.5.
 //   3-4 tokens, one round: 4096 x 12288 14.5 -> 14.1, past that 4096 x 14336
 //     16.3 -> 17.0; 6144 x 2048 7.1 -> 5.9, 4096 x 1536 5.5 -> 4.9, below that
 //     1024 x 768 4.4 -> 4.4 and, two tiles per wave, SwiGLU 8192 x 1024 6.0 -> 6.2.
@@ -383,8 +383,8 @@ hipError_t w8a16_batch(const uint16_t* x, int64_t ldx, const uint8_t* w, int64_t
 // tile, by K, and by how many workgroups each CU runs, half as much with two
 // weight tiles per activation load. The lines lie where 4200 timed pairs on
 // MI355X cross (17-64 tokens, 15 row lengths, 16 widths; rows as they are ->
-// packed, us, graphs over 1 GiB of rotated weights, N x K; kept, the packed side is
-// at most 6 % slower anywhere and 1.4 % off the faster side on average):
+// packed, us, graphs over 1 GiB of rotated weights, N x K); the side they take is at
+// most 6 % slower where it packs, and 1.4 % off the faster one on average:
 //   17-32 tokens, several rounds: 10240 x 8192 at 17 / 24 33.2 / 40.3 -> 34.4 /
 //     34.4, 12288 x 2048 at 24 / 28 12.5 / 13.6 -> 12.9 / 12.9, two tiles per
 //     wave 16384 x 4096 at 20 / 24 19.7 / 20.9 -> 20.4 / 20.5, short rows 16384 x

@@ -165,10 +165,13 @@ def _row_major(codes: torch.Tensor) -> tuple[torch.Tensor, int]:
     """Row-major codes and their row stride for the C ABI, where a stride of 0
     names the packed layouts: one row broadcast by ``expand`` is copied out to
     its rows, and a single row passes its length."""
-    if not _rows_aligned(codes, 1):
-        codes = codes.contiguous()
-    if codes.stride(0) == 0 and codes.shape[0] > 1:
+    ld, unit = codes.stride()
+    if ld and unit == 1 and ld % 16 == 0 and codes.data_ptr() % 16 == 0:
+        return codes, ld
+    if ld == 0 and codes.shape[0] > 1:
         codes = codes.clone(memory_format=torch.contiguous_format)
+    elif not _rows_aligned(codes, 1):
+        codes = codes.contiguous()
     return codes, codes.stride(0) or codes.shape[1]
 
 
